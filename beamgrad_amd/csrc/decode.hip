@@ -359,35 +359,45 @@ hipError_t launch_decode(const DecodeParams& p0, const DecodeLayout& L, hipStrea
     e = launch_clear_ranges(clear, stream);
     if (e == hipSuccess) e = hipEventRecord(aux->start, stream);
     // A persistent row pass is launched first: its grid leaves the select
-    // pass's CUs free. A row pass of one workgroup per row would fill every
-    // CU before the select pass's workgroups are placed, so the select pass
-    // goes first there, split in two launches (DecodeParams::claimed): the
-    // early one before the row pass takes the examples whose first row comes
-    // within 200 us, the late one after it takes the rest. The streams are
-    // not guaranteed to run at once (HIP maps streams onto a few hardware
-    // queues, shared once there are more streams), and no select-pass wait
-    // may depend on a launch submitted after it.
+    // pass's CUs free, and the select pass follows on the second stream. A
+    // row pass of several workgroups per CU would fill every CU before the
+    // select pass's workgroups are placed (a select pass that holds its CUs
+    // then starts only as the row pass ends: 16 x 64 x 64 x 32000 f32
+    // log-probs 2.5 ms instead of 1.6), so the select pass goes first there,
+    // on the caller's own stream right behind the clear, and the row pass on
+    // the second stream, whose wait for the clear lets the select pass in
+    // ahead of it. The select pass is split in two launches
+    // (DecodeParams::claimed): the early one before the row pass takes the
+    // examples whose first row comes within 200 us, the late one after it
+    // takes the rest. The streams are not guaranteed to run at once (HIP maps
+    // streams onto a few hardware queues, shared once there are more
+    // streams), and no select-pass wait may depend on a launch submitted
+    // after it.
     p.select_hold = hold ? 1 : 0;
-    if (e == hipSuccess && persistent) e = launch_row_pass(p, stream);
-    if (e == hipSuccess) e = hipStreamWaitEvent(aux->stream, aux->start, 0);
     if (persistent) {
+        if (e == hipSuccess) e = launch_row_pass(p, stream);
+        if (e == hipSuccess) e = hipStreamWaitEvent(aux->stream, aux->start, 0);
         if (e == hipSuccess) e = launch_select(p, L.sel, aux->stream);
+        if (e == hipSuccess) e = hipEventRecord(aux->done, aux->stream);
+        if (e == hipSuccess) e = hipStreamWaitEvent(stream, aux->done, 0);
     } else {
         DecodeParams early = p;
         early.claimed = claimed;
         early.early = 1;
         early.early_ticks = 20000;  // 200 us of the 100 MHz counter
-        if (e == hipSuccess) e = launch_select(early, L.sel, aux->stream);
-        if (e == hipSuccess) e = launch_row_pass(p, stream);
+        if (e == hipSuccess) e = launch_select(early, L.sel, stream);
+        if (e == hipSuccess) e = hipStreamWaitEvent(aux->stream, aux->start, 0);
+        if (e == hipSuccess) e = launch_row_pass(p, aux->stream);
+        if (e == hipSuccess) e = hipEventRecord(aux->done, aux->stream);
+        if (e == hipSuccess) e = hipStreamWaitEvent(stream, aux->done, 0);
         DecodeParams late = early;
         late.early = 0;
-        if (e == hipSuccess) e = launch_select(late, L.sel, aux->stream);
+        if (e == hipSuccess) e = launch_select(late, L.sel, stream);
     }
-    if (e == hipSuccess) e = hipEventRecord(aux->done, aux->stream);
-    if (e == hipSuccess) e = hipStreamWaitEvent(stream, aux->done, 0);
     if (e == hipSuccess) {
         *fault = p.fault;
-        t_last_overlap = LastOverlap{p.fault, aux, aux->stream, aux->epoch};
+        t_last_overlap =
+            persistent ? LastOverlap{p.fault, aux, aux->stream, aux->epoch} : LastOverlap{};
     }
     return e;
 }
