@@ -253,6 +253,16 @@ void set_pool(DecodeParams& p, const PoolOutputs* pool) {
     p.pool_flp = pool->from_logprob;
 }
 
+// The decode's layout; beyond 64 beams, the one without shortlists where the
+// caller's workspace (or the static scratch) has room for no more.
+DecodeLayout fitting_layout(const void* workspace, int64_t workspace_bytes, int B, int T, int K, int V, bool cons,
+                            bool step_mode, int prefix_stride, int keep) {
+    const DecodeLayout L = decode_layout(B, T, K, V, cons, step_mode, prefix_stride, keep);
+    if (!workspace || workspace_bytes >= static_cast<int64_t>(L.total)) return L;
+    const DecodeLayout small = decode_layout(B, T, K, V, cons, step_mode, prefix_stride, keep, false);
+    return workspace_bytes >= static_cast<int64_t>(small.total) ? small : L;
+}
+
 int decode_common(const void* inputs, int data_type, int from_logits, const DBSCudaDecodeArgs* args,
                   const DBSCudaSearchOptions* options, const uint8_t* banned_pe, const DBSCudaDecodeOutputs* outputs,
                   float* row_lse, void* workspace, int64_t workspace_bytes, void* stream_ptr,
@@ -267,8 +277,8 @@ int decode_common(const void* inputs, int data_type, int from_logits, const DBSC
     const int pool_mult = pool ? pool->mult : 0;
     if (pool_mult < 0 || static_cast<int64_t>(pool_mult) * a.beam_size > DBS_CUDA_MAX_BEAM)
         return DBS_CUDA_STATUS_INVALID_ARGUMENT;
-    const DecodeLayout L =
-        decode_layout(a.batch_size, a.steps, a.beam_size, a.vocab_size, cons, false, 0, pool_mult * a.beam_size);
+    const DecodeLayout L = fitting_layout(workspace, workspace_bytes, a.batch_size, a.steps, a.beam_size, a.vocab_size,
+                                          cons, false, 0, pool_mult * a.beam_size);
     bool too_small = false;
     Scratch scratch;
     hipError_t e = scratch.acquire(workspace, workspace_bytes, L.total, stream, &too_small);
@@ -345,8 +355,8 @@ int step_common(const void* inputs, int data_type, int from_logits, const DBSCud
     const int pool_mult = pool ? pool->mult : 0;
     if (pool_mult < 0 || static_cast<int64_t>(pool_mult) * a.beam_size > DBS_CUDA_MAX_BEAM)
         return DBS_CUDA_STATUS_INVALID_ARGUMENT;
-    DecodeLayout L = decode_layout(a.batch_size, 1, a.beam_size, a.vocab_size, cons, true, state->prefix_stride,
-                                   pool_mult * a.beam_size);
+    DecodeLayout L = fitting_layout(workspace, workspace_bytes, a.batch_size, 1, a.beam_size, a.vocab_size, cons, true,
+                                    state->prefix_stride, pool_mult * a.beam_size);
     if (row_mask) L.M = 0;  // filtered rows are read in full
     bool too_small = false;
     Scratch scratch;
@@ -678,10 +688,10 @@ DBS_CUDA_EXPORT int dbs_hip_decode_noalloc(const void* inputs, int data_type, in
         return DBS_CUDA_STATUS_INVALID_ARGUMENT;
     if (!valid_options(options, *args)) return DBS_CUDA_STATUS_INVALID_ARGUMENT;
     const DBSCudaDecodeArgs& a = *args;
-    const DecodeLayout L =
-        decode_layout(a.batch_size, a.steps, a.beam_size, a.vocab_size, constrained(a), false, 0);
-    if (L.total > static_cast<size_t>(DBS_HIP_NOALLOC_SCRATCH_BYTES)) return DBS_HIP_STATUS_SCRATCH_LIMIT;
     void* ws = nullptr;
+    const DecodeLayout L = fitting_layout(&ws, DBS_HIP_NOALLOC_SCRATCH_BYTES, a.batch_size, a.steps, a.beam_size,
+                                          a.vocab_size, constrained(a), false, 0, 0);
+    if (L.total > static_cast<size_t>(DBS_HIP_NOALLOC_SCRATCH_BYTES)) return DBS_HIP_STATUS_SCRATCH_LIMIT;
     const hipError_t e = scratch_address(&ws);
     if (e != hipSuccess) {
         (void)hipGetLastError();

@@ -102,13 +102,18 @@ __global__ void check_examples_kernel(const int32_t* steps, const int32_t* beams
 }  // namespace
 
 DecodeLayout decode_layout(int B, int T, int K, int V, bool constrained, bool step_mode, int prefix_stride,
-                           int keep) {
+                           int keep, bool wide_lists) {
     DecodeLayout L{};
     // Shortlist length: the candidates kept per step (K, or the relaxed
     // pool) plus a margin, while the row pass can pick its threshold from the
-    // row's 256 lane maxima; more rescan every row.
+    // row's 256 lane maxima. More beams than that keep the same 80 entries per
+    // row: K rows share the K selections, and only the first steps, whose
+    // candidates come from a few rows, read rows in full (select_kernel's WIDE;
+    // 4 x 8 x 256 x 32000 f32 log-probs: 38.7 ms reading every row in full,
+    // 0.49 ms with the lists, the row pass alone 0.18). Larger relaxed pools rescan every row, and so does a decode whose
+    // caller's workspace has no room for the lists (wide_lists false).
     const int kept = keep > 0 ? keep : K;
-    int M = kept <= 64 ? ((kept + 16 + 7) / 8) * 8 : 0;
+    int M = kept <= 64 ? ((kept + 16 + 7) / 8) * 8 : (kept == K && wide_lists ? 80 : 0);
     if (const char* env = std::getenv("DBS_HIP_SHORTLIST")) {
         // testing knob: 0 forces full rescans, a small value forces fallbacks
         const int m = std::atoi(env);

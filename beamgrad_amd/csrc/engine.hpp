@@ -178,8 +178,9 @@ struct DecodeLayout {
 
 // keep: candidates a step keeps per example (0: K; the relaxed pool keeps
 // more), which sizes the shortlists and the select pass's collector.
+// wide_lists false: no shortlists beyond 64 beams (a small workspace).
 DecodeLayout decode_layout(int B, int T, int K, int V, bool constrained, bool step_mode, int prefix_stride,
-                           int keep = 0);
+                           int keep = 0, bool wide_lists = true);
 SelectLayout select_layout(int B, int T, int K, int M, bool constrained, bool step_mode, int prefix_cap,
                            int keep = 0);
 
@@ -212,6 +213,13 @@ hipError_t launch_row_logprob(const DecodeParams& p, int64_t rows, hipStream_t s
 extern std::atomic<int> g_row_pass_kind;  // dbs_hip_set_row_pass
 hipError_t launch_row_pipe(const DecodeParams& p, int64_t rows, hipStream_t stream);
 hipError_t launch_select(const DecodeParams& p, const SelectLayout& L, hipStream_t stream);
+// The kernels of one input type (0 f32, 1 f16, 2 bf16), and their counters.
+template <int DT>
+hipError_t launch_select_dtype(const DecodeParams& p, const SelectLayout& L, hipStream_t stream);
+template <int DT>
+hipError_t rescan_counter_dtype(int reset, unsigned long long* value);
+template <int DT>
+hipError_t wait_timeout_counter_dtype(int reset, unsigned long long* value);
 // The select pass runs one wavefront per example (narrow, unconstrained
 // decodes with shortlists) instead of one workgroup; dbs_hip_set_select_pass
 // (g_select_kind 1) keeps the workgroup pass.

@@ -10,9 +10,16 @@
 // the selection exact: a row whose bound could still beat the K-th selected
 // candidate is rescanned in full from HBM. The trace, the beam state and the
 // prefixes advance as in reference src/decoder.cpp:122-187, 314-350.
+//
+// Included by one translation unit per input type (select_f32.hip,
+// select_f16.hip, select_bf16.hip), which instantiates the kernels of its
+// type; select.hip plans and dispatches.
+#pragma once
+
 #include <hip/hip_runtime.h>
 
 #include "device_common.hpp"
+#include "select_plan.hpp"
 
 namespace dbs_hip {
 
@@ -22,8 +29,6 @@ namespace {
 __device__ unsigned long long g_rescanned_rows;
 // Waits for a step of the overlapped decode that gave up (should stay 0).
 __device__ unsigned long long g_wait_timeouts;
-
-constexpr int kStageTags = 8;  // tagged shortlist loads per thread in flight (workgroup pass, overlapped decode)
 
 // Overlapped decode: waits until the row pass has counted every row of
 // example b's step t: one at step 0, else one per beam of the example (the
@@ -81,18 +86,46 @@ __device__ __forceinline__ bool wait_tagged(const DecodeParams& p, const uint32_
     return true;
 }
 
-constexpr int kRescanBuf = 512;   // candidates of one rescanned row kept before falling back
-constexpr int kRescanPerThread = 16;
-constexpr int kTauHead = 2;       // entries per row behind the second tau bound
-constexpr int kWideBeam = 16;     // beams from which the wide-beam paths pay off
-constexpr int kPfRegs = 12;       // 16-byte prefetch registers per thread (K * M <= 6144)
-constexpr int kSigWordsMax = 256;  // words of a beam's prefix signature (8192 bits; 2048 when LDS is short)
-constexpr int kScoreFilterMaxK = 32;  // beams up to which a rank compaction first ranks by score alone
+// The key of the M-th largest of n keys in LDS (n a multiple of kSelectThreads,
+// at most 2048; zero keys pad), its low LOW bits zero (at least M keys reach
+// it), in every thread of the workgroup: the radix select of mth_largest_key,
+// each wavefront counting its quarter, the counts exchanged through part [8]
+// (one barrier a bit). The caller's barrier precedes it.
+template <int LOW>
+__device__ __forceinline__ uint32_t mth_largest_wg(const uint32_t* key, int n, int M, int32_t* part) {
+    constexpr int kPer = 2048 / kSelectThreads;
+    const int tid = static_cast<int>(threadIdx.x), w = tid >> 6;
+    uint32_t k[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) k[u] = u * kSelectThreads < n ? key[u * kSelectThreads + tid] : 0u;
+    uint32_t prefix = 0;
+    int need = M;
+#pragma unroll 1
+    for (int bit = 31; bit >= LOW; --bit) {
+        const uint32_t want = (prefix >> bit) | 1u;
+        int c = 0;
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) c += __popcll(__ballot((k[u] >> bit) == want));
+        int32_t* const slot = part + 4 * (bit & 1);
+        if ((tid & 63) == 0) slot[w] = c;
+        lds_barrier();
+        const int4 all = *reinterpret_cast<const int4*>(slot);
+        c = __builtin_amdgcn_readfirstlane(all.x + all.y + all.z + all.w);
+        if (c >= need) {
+            prefix |= 1u << bit;
+        } else {
+            need -= c;
+        }
+    }
+    return prefix;
+}
 
 struct Lds {
     Cand* buf;        // [sort_cap] the collector
-    Cand* rbuf;       // [kRescanBuf] one rescanned row's candidates
-    uint4* key;       // [2 * kRankMax] candidate keys of a rank compaction (kRankMax used)
+    int32_t* rbuf;    // [kRescanTokens] tokens gathered from one rescanned row
+    uint4* key;       // [2 * kRankMax] candidate keys of a rank compaction (kRankMax used; WIDE: [4 * kRankMax])
+    bool wide;        // more than kListBeams beams
+    int32_t* rank;    // [4 * kRankMax] (WIDE) ranks of a compaction
     int32_t* part;    // [kSelectThreads] partial ranks (or score keys)
     int32_t* surv;    // [64] candidates left by the score pass of a rank compaction
     int32_t* nsurv;   // [1] how many
@@ -247,10 +280,6 @@ __device__ __forceinline__ void sort_cands(Cand* buf, int np) {
     }
 }
 
-// Collector sizes up to this are compacted by a parallel rank (larger ones by
-// the bitonic sort).
-constexpr int kRankMax = kSelectThreads;
-
 // The candidate at collector index idx as a 96-bit integer that is larger
 // exactly when the candidate comes earlier in the total order, least
 // significant word first: (parent, token) as parent * V + token (asc), raw,
@@ -404,11 +433,89 @@ __device__ __forceinline__ void compact_by_rank(Lds& s, State& st, int K, int n)
     lds_barrier();
 }
 
+// The same for n <= 1024 candidates (more than 64 beams: the collector holds K
+// to about 2 K of them). Every wavefront keeps all the keys, up to 16 a lane,
+// and counts a quarter of the others against them, so that a key is read from
+// LDS once, not once per wavefront (a broadcast read of 16 bytes costs the
+// LDS as much as 64 distinct ones: with each wavefront counting its own
+// candidates, n = 290 took 12.5 us). Bound by the compares of all pairs, n^2 /
+// 16 cycles.
+constexpr int kWideKeys = kWideRank * kSelectThreads / 64;  // keys per lane
+__device__ __forceinline__ void compact_wide(Lds& s, State& st, int K, int n) {
+    const int tid = static_cast<int>(threadIdx.x), lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    Cand c[kWideRank];
+#pragma unroll
+    for (int u = 0; u < kWideRank; ++u) {
+        const int i = tid + u * kSelectThreads;
+        if (u * kSelectThreads < n) {
+            uint4 key = make_uint4(0u, 0u, 0u, 0u);  // below every key
+            if (i < n) {
+                c[u] = s.buf[i];
+                key = cand_key(c[u], i, s.V);
+            }
+            s.key[i] = key;
+            s.rank[i] = 0;
+        }
+    }
+    lds_barrier();
+    uint32_t k0[kWideKeys], k1[kWideKeys], k2[kWideKeys];
+    int rank[kWideKeys];
+#pragma unroll
+    for (int u = 0; u < kWideKeys; ++u) {
+        rank[u] = 0;
+        k0[u] = k1[u] = k2[u] = 0u;
+        if (64 * u < n) {
+            const uint4 key = s.key[64 * u + lane];
+            k0[u] = key.x;
+            k1[u] = key.y;
+            k2[u] = key.z;
+        }
+    }
+    const int span = ((n + 15) >> 4) << 2;  // a quarter, in fours (the keys past n are zero)
+    const int j1 = min(n, (w + 1) * span);
+#pragma unroll 1
+    for (int j = w * span; j < j1; j += 4) {
+        uint4 x[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) x[v] = s.key[j + v];
+#pragma unroll
+        for (int u = 0; u < kWideKeys; u += 2) {
+            if (64 * u < n) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    count_above96(rank[u], k0[u], k1[u], k2[u], x[v].x, x[v].y, x[v].z);
+                    count_above96(rank[u + 1], k0[u + 1], k1[u + 1], k2[u + 1], x[v].x, x[v].y, x[v].z);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kWideKeys; ++u)
+        if (64 * u + lane < n) atomicAdd(&s.rank[64 * u + lane], rank[u]);
+    lds_barrier();
+#pragma unroll
+    for (int u = 0; u < kWideRank; ++u) {
+        const int i = tid + u * kSelectThreads;
+        if (i < n) {
+            const int r = s.rank[i];
+            if (r < K) s.buf[r] = c[u];
+            if (r == K - 1 && before(c[u], st.thr)) st.thr = c[u];
+        }
+    }
+    if (tid == 0) st.count = n < K ? n : K;
+    lds_barrier();
+}
+
 // Sorts the collected candidates, keeps the best K, and raises the admission
 // threshold to the K-th kept one when that is better.
 __device__ __forceinline__ void compact(Lds& s, State& st, int K) {
     lds_barrier();
     const int n = __builtin_amdgcn_readfirstlane(st.count);
+    if (s.wide && n <= kWideRank * kRankMax) {
+        compact_wide(s, st, K, n);
+        return;
+    }
     if (n <= kRankMax) {
         compact_by_rank(s, st, K, n);
         return;
@@ -440,9 +547,20 @@ __device__ __forceinline__ void end_round(Lds& s, State& st, int K, int sort_cap
 }
 
 // Every candidate of row `row` (beam k) that does not rank after the
-// threshold: gathered into the rescan buffer in one sweep, then offered to the
-// collector. A buffer overflow (a row with very many candidates at the
-// threshold) falls back to offering round by round.
+// threshold: a sweep over the row gathers the tokens whose score could reach
+// it, then their candidates are offered to the collector. With no threshold
+// yet, or more tokens than the buffer holds (the first step's one row of a
+// wide beam, a step whose threshold is still low), a sweep takes the best
+// score of 4 slices of the row per thread first: the keep-th best of those
+// 1024 is reached by at least `keep` candidates of this row, so the tokens
+// below it are left out (of 32000 at keep = 256 some 300 remain; each 256 past
+// the collector's room cost a sort before). More at that score than the buffer
+// holds: offered round by round.
+// One workgroup reads the row, so a sweep is bound by the latency of its
+// batches (kRescanPerThread loads in flight per thread, about 2 us each), and
+// the full candidate test is made once per gathered token: inlined for every
+// element of a batch it is more code than the instruction cache holds (80 us a
+// sweep of 32000).
 template <int DT, bool LOGITS>
 __device__ __forceinline__ void rescan_row(const DecodeParams& p, Lds& s, State& st, int b, int k, int64_t row, float lse,
                            float praw, float inv_pen, int new_len, const PrefixView& pre, int sort_cap, int keep) {
@@ -451,60 +569,119 @@ __device__ __forceinline__ void rescan_row(const DecodeParams& p, Lds& s, State&
     const int tid = static_cast<int>(threadIdx.x);
     const size_t esz = DT == 0 ? 4 : 2;
     const char* base = static_cast<const char*>(p.x) + static_cast<size_t>(row) * static_cast<size_t>(V) * esz;
-    if (tid == 0) {
-        st.rcount = 0;
-        st.overflow = 0;
-    }
-    lds_barrier();
     const Cand thr = st.thr;
-    for (int v0 = 0; v0 < V; v0 += kSelectThreads * kRescanPerThread) {
+    float least = -kInf;
+    const bool plain = !p.banned && !p.banned_pe && !p.row_mask && !mask_eos && !p.constrained;
+    // token v's candidate, unless it is excluded, ranks after the threshold or
+    // lies below `least`
+    auto candidate = [&](int v, Cand& c) -> bool {
+        const float x = load_one<DT>(base, v);
+        const float lp = LOGITS ? x - lse : x;
+        if (!(lp < kInf) || lp == -kInf) return false;
+        if (static_masked(p, b, v, mask_eos)) return false;
+        if (p.row_mask && gload(p.row_mask, row * V + v)) return false;
+        if (!make_cand(p, s, pre, k, praw, inv_pen, v, new_len, lp, c)) return false;
+        return !(c.score < least) && !before(thr, c);
+    };
+    // A batch's scores, penalties apart (they only lower a candidate); NaN,
+    // which passes no test, where there is no finite entry.
+    auto scan = [&](int v0, float (&score)[kRescanPerThread]) __attribute__((always_inline)) {
         float xs[kRescanPerThread];
 #pragma unroll
-        for (int j = 0; j < kRescanPerThread; ++j) {
+        for (int j = 0; j < kRescanPerThread; ++j) {  // every load made, from a clamped index
             const int v = v0 + j * kSelectThreads + tid;
-            xs[j] = v < V ? load_one<DT>(base, v) : -kInf;
+            xs[j] = load_one<DT>(base, v < V ? v : V - 1);
         }
 #pragma unroll
         for (int j = 0; j < kRescanPerThread; ++j) {
-            const int v = v0 + j * kSelectThreads + tid;
             const float lp = LOGITS ? xs[j] - lse : xs[j];
-            if (v >= V || !(lp < kInf) || lp == -kInf) continue;
-            const float raw0 = praw + lp;
-            const Cand c0{raw0 * inv_pen, raw0, k, v, new_len, 1};
-            if (before(thr, c0)) continue;  // penalties only lower a candidate
-            if (static_masked(p, b, v, mask_eos)) continue;
-            if (p.row_mask && gload(p.row_mask, row * V + v)) continue;
-            Cand c;
-            if (!make_cand(p, s, pre, k, praw, inv_pen, v, new_len, lp, c)) continue;
-            if (before(thr, c)) continue;
-            const int slot = atomicAdd(&st.rcount, 1);
-            if (slot < kRescanBuf) s.rbuf[slot] = c;
-            else st.overflow = 1;
+            const bool in = v0 + j * kSelectThreads + tid < V && lp < kInf && lp > -kInf;
+            score[j] = in ? (praw + lp) * inv_pen : __builtin_nanf("");
         }
-    }
-    lds_barrier();
-    if (!st.overflow) {
-        const int n = st.rcount;
-        for (int r0 = 0; r0 < n; r0 += kSelectThreads) {
-            if (r0 + tid < n) offer(s, st, s.rbuf[r0 + tid]);
-            end_round(s, st, keep, sort_cap);
+    };
+    int32_t* const tokens = s.rbuf;
+#pragma unroll 1
+    for (int attempt = thr.parent < 0 ? 1 : 0; attempt < 2; ++attempt) {
+        lds_barrier();  // (the buffer and the flags are free)
+        if (attempt == 1) {
+            float best[4] = {-kInf, -kInf, -kInf, -kInf};
+#pragma unroll 1
+            for (int v0 = 0; v0 < V; v0 += kSelectThreads * kRescanPerThread) {
+                float score[kRescanPerThread];
+                scan(v0, score);
+                if (plain) {
+#pragma unroll
+                    for (int j = 0; j < kRescanPerThread; ++j) best[j & 3] = fmaxf(best[j & 3], score[j]);
+                } else {
+                    uint32_t pass = 0;
+#pragma unroll
+                    for (int j = 0; j < kRescanPerThread; ++j) pass |= (score[j] > best[j & 3] ? 1u : 0u) << j;
+                    while (pass != 0) {
+                        const int j = __ffs(static_cast<int>(pass)) - 1;
+                        pass &= pass - 1;
+                        Cand c;
+                        if (!candidate(v0 + j * kSelectThreads + tid, c)) continue;
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) best[u] = (j & 3) == u ? fmaxf(best[u], c.score) : best[u];
+                    }
+                }
+            }
+            uint32_t* const slice = reinterpret_cast<uint32_t*>(s.rbuf);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) slice[u * kSelectThreads + tid] = ordered_key(best[u]);
+            lds_barrier();
+            const float at = key_value(mth_largest_wg<0>(slice, 4 * kSelectThreads, keep, s.surv));
+            lds_barrier();  // (the slices are read: the buffer is free)
+            least = at;
         }
-        return;
-    }
-    // very many candidates at the threshold: offer the row round by round
-    for (int v0 = 0; v0 < V; v0 += kSelectThreads) {
-        const int v = v0 + tid;
-        if (v < V) {
-            const float x = load_one<DT>(base, v);
-            const float lp = LOGITS ? x - lse : x;
-            if ((lp < kInf) && lp != -kInf && !static_masked(p, b, v, mask_eos) &&
-                !(p.row_mask && gload(p.row_mask, row * V + v))) {
-                Cand c;
-                if (make_cand(p, s, pre, k, praw, inv_pen, v, new_len, lp, c)) offer(s, st, c);
+        if (tid == 0) st.rcount = 0;
+        lds_barrier();
+        const float floor_score = fmaxf(least, thr.score);
+#pragma unroll 1
+        for (int v0 = 0; v0 < V; v0 += kSelectThreads * kRescanPerThread) {
+            float score[kRescanPerThread];
+            scan(v0, score);
+            uint32_t pass = 0;
+#pragma unroll
+            for (int j = 0; j < kRescanPerThread; ++j) pass |= (score[j] >= floor_score ? 1u : 0u) << j;
+            while (pass != 0) {
+                const int j = __ffs(static_cast<int>(pass)) - 1;
+                pass &= pass - 1;
+                const int slot = atomicAdd(&st.rcount, 1);
+                if (slot < kRescanTokens) tokens[slot] = v0 + j * kSelectThreads + tid;
             }
         }
+        lds_barrier();
+        const int n = st.rcount;
+        if (n <= kRescanTokens) {
+            for (int r0 = 0; r0 < n; r0 += kSelectThreads) {
+                Cand c;
+                if (r0 + tid < n && candidate(tokens[r0 + tid], c)) offer(s, st, c);
+                end_round(s, st, keep, sort_cap);
+            }
+            return;
+        }
+    }
+    for (int v0 = 0; v0 < V; v0 += kSelectThreads) {
+        const int v = v0 + tid;
+        Cand c;
+        if (v < V && candidate(v, c)) offer(s, st, c);
         end_round(s, st, keep, sort_cap);
     }
+}
+
+// Entry i of a shortlist in global memory (more than 64 beams: the lists are
+// not staged), within its row's count. Overlapped decode: waited for while
+// not written yet; a wait that gives up marks the example and reads as -inf.
+__device__ __forceinline__ ShortEntry list_entry(const DecodeParams& p, State& st, int64_t row, int i) {
+    const uint32_t* src = reinterpret_cast<const uint32_t*>(p.shortlist + row * p.M + i);
+    if (p.step_done == nullptr) return p.shortlist[row * p.M + i];
+    uint32_t lo = 0, hi = 0;
+    if (!read_tagged(src, lo, hi) && !wait_tagged(p, src, lo, hi)) {
+        atomicOr(&st.gave_up, 1);
+        return ShortEntry{-kInf, 0};
+    }
+    return ShortEntry{bits_f32(lo), static_cast<int32_t>(hi) - 1};
 }
 
 // PF: the next step's RowInfo and shortlists are prefetched into registers
@@ -515,7 +692,14 @@ __device__ __forceinline__ void rescan_row(const DecodeParams& p, Lds& s, State&
 // before a row pass of one workgroup per row, it keeps its CUs to itself
 // (registers it never uses; its own occupancy, one wavefront per SIMD, is
 // unchanged).
-template <int DT, bool LOGITS, bool PF, bool HOLD = false>
+// WIDE: more than kListBeams beams. The shortlists (shorter than the beams are
+// many) stay in global memory: each thread keeps the head of its beams' lists
+// in LDS, tau is the K-th largest raw of the heads, and each beam's prefix
+// that reaches tau goes to the collector. Most rows give one or two of the K
+// selected candidates, so a step reads a few entries per row; the rows that
+// give more than their list holds (the first step's one row, a few of the
+// next) fail the exactness check and are read in full.
+template <int DT, bool LOGITS, bool PF, bool HOLD = false, bool WIDE = false>
 __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, SelectLayout L) {
     if constexpr (HOLD) asm volatile("" ::: "a255");
     extern __shared__ __align__(16) unsigned char smem[];
@@ -530,12 +714,20 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, 
     const int SL = sl_stride(K, M);
     const int b = static_cast<int>(blockIdx.x);
     const int tid = static_cast<int>(threadIdx.x);
+    // WIDE: entries of each list's head in LDS, the most of 8, 4, 2 that keep
+    // K of them within kHeads (8 leave 1.2 to 1.5 K candidates at tau, 2 leave
+    // 2 to 4 K: each list gives few, the best ones up to 80); 0 without lists
+    constexpr int kHeadMax = WIDE ? 8 : 1;
+    const int hsh = K <= kHeads / 8 ? 3 : (K <= kHeads / 4 ? 2 : 1);
+    const int H = WIDE && M >= 8 ? 1 << hsh : 0;
 
     Lds s;
     s.buf = reinterpret_cast<Cand*>(smem + L.off_buf);
-    s.rbuf = reinterpret_cast<Cand*>(smem + L.off_rbuf);
+    s.rbuf = reinterpret_cast<int32_t*>(smem + L.off_rbuf);
     s.key = reinterpret_cast<uint4*>(smem + L.off_key);
-    s.part = reinterpret_cast<int32_t*>(smem + L.off_key + sizeof(uint4) * 2 * kRankMax);
+    s.part = reinterpret_cast<int32_t*>(smem + L.off_key + sizeof(uint4) * (WIDE ? 4 : 2) * kRankMax);
+    s.wide = WIDE;
+    s.rank = WIDE ? s.part + kSelectThreads + 64 + 4 : nullptr;
     s.surv = s.part + kSelectThreads;
     s.nsurv = s.surv + 64;
     float* f = reinterpret_cast<float*>(smem + L.off_f32);
@@ -684,7 +876,26 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, 
             const bool carried = live && eos_b >= 0 && s.ended[k];
             int cnt = -2;
             float bound = -kInf;
+            // WIDE: the head of the beam's list, loaded with its RowInfo, every
+            // load from a clamped entry (those past the row's count are not
+            // used)
+            uint32_t elo[kHeadMax], ehi[kHeadMax];
             if (live && !carried) {
+                if constexpr (WIDE) {
+                    if (H > 0) {
+                        const uint32_t* esrc = reinterpret_cast<const uint32_t*>(p.shortlist + (trace0 + k) * M);
+#pragma unroll
+                        for (int u = 0; u < kHeadMax; ++u) {
+                            const int i = u < H ? u : H - 1;
+                            if (coherent) {
+                                (void)read_tagged(esrc + 2 * i, elo[u], ehi[u]);
+                            } else {
+                                elo[u] = esrc[2 * i];
+                                ehi[u] = esrc[2 * i + 1];
+                            }
+                        }
+                    }
+                }
                 RowInfo info;
                 if (have_pf) {
                     __builtin_memcpy(&info, &pf_info, sizeof(info));  // k == tid
@@ -717,6 +928,25 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, 
                 bound = info.bound;
                 s.nraw[k] = info.lse;  // the row's logsumexp, kept for a rescan
             }
+            if constexpr (WIDE) {
+                if (H > 0) {
+#pragma unroll
+                    for (int u = 0; u < kHeadMax; ++u) {
+                        if (u >= H) break;
+                        ShortEntry e{-kInf, 0};
+                        if (u < cnt) {
+                            const uint32_t* esrc = reinterpret_cast<const uint32_t*>(p.shortlist + (trace0 + k) * M + u);
+                            if (coherent && ehi[u] == 0u && !wait_tagged(p, esrc, elo[u], ehi[u])) {
+                                atomicOr(&st.gave_up, 1);
+                                elo[u] = f32_bits(-kInf);
+                                ehi[u] = 1;
+                            }
+                            e = ShortEntry{bits_f32(elo[u]), static_cast<int32_t>(coherent ? ehi[u] - 1u : ehi[u])};
+                        }
+                        s.sl[k * H + u] = e;
+                    }
+                }
+            }
             s.rcount[k] = cnt;
             s.rbound[k] = bound;
             if (p.constrained && p.ngram > 1) s.nblk[k] = 0;
@@ -729,7 +959,9 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, 
                 continue;
             }
         }
-        if (have_pf) {
+        if constexpr (WIDE) {
+            // the lists stay where they are
+        } else if (have_pf) {
             const int n4 = K * M / 2;
 #pragma unroll
             for (int u = 0; u < kPf; ++u) {
@@ -836,7 +1068,26 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, 
         }
         // a forced step (uniform over the workgroup): no shortlist is used
         const int forced = p.forced ? gload(p.forced, static_cast<int64_t>(b) * T + t) : -1;
-        if (p.use_tau && forced < 0) {
+        if constexpr (WIDE) {
+            // tau: the K-th largest raw of the rows' heads (to its 20 highest
+            // bits, rounded down), reached by at least K real candidates
+            if (H > 0 && p.use_tau && forced < 0) {
+                const int nv = K * H;
+                uint32_t* vk = reinterpret_cast<uint32_t*>(s.key);
+                for (int q = tid; q < ((nv + 255) & ~255); q += kSelectThreads) {
+                    const int k = q >> hsh;
+                    vk[q] = q < nv ? ordered_key(q - k * H < s.rcount[k] ? s.raw[k] + s.sl[q].lp : -kInf) : 0u;
+                }
+                lds_barrier();
+                const float tau = key_value(mth_largest_wg<12>(vk, (nv + 255) & ~255, K, s.surv));
+                if (tid == 0) {
+                    st.tau = tau > -kInf ? tau : -kInf;  // (a key cut below -inf's reads as NaN)
+                    st.rcount = 0;
+                    st.overflow = 0;
+                }
+                lds_barrier();
+            }
+        } else if (p.use_tau && forced < 0) {
             // Lower bounds of the K-th best expanded raw (unconstrained: raw =
             // fl(p + lp), monotone in lp; every beam expanded has the same
             // length, so this step's shortlisted candidates rank by raw).
@@ -926,7 +1177,7 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, 
         }
         // (at most K offers: the first round of shortlisted offers joins them
         // unless the one-pass path below needs the count)
-        if (M > 0 && p.use_tau && K >= kWideBeam && forced < 0) end_round(s, st, KP, L.sort_cap);
+        if (!WIDE && M > 0 && p.use_tau && K >= kWideBeam && forced < 0) end_round(s, st, KP, L.sort_cap);
 
         // Shortlisted candidates. Unconstrained wide beams: few reach tau, and
         // when they fit the collector beside what it holds, they are offered
@@ -935,7 +1186,64 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, 
         // are a prefix of it: one thread per beam measures its prefix, then
         // offers it.
         bool one_pass = false;
-        if (M > 0 && p.use_tau && K >= kWideBeam && forced < 0) {
+        if constexpr (WIDE) {
+            if (H > 0 && p.use_tau && forced < 0) {
+                // Each beam's entries that reach tau go to the collector, as
+                // long as they fit: those of its head by the beam's thread,
+                // and where the whole head does, the rest of its list by a
+                // wavefront, one entry a lane (a thread walking a list of 80
+                // took 40 us a step).
+                lds_barrier();  // the carried beams are in
+                const float tau = st.tau;
+                const int base = st.count;
+                int32_t* const found = s.nlen;  // the beams whose head does not hold them all (free until the selection)
+                auto put = [&](int slot, int k, const ShortEntry& e) __attribute__((always_inline)) {
+                    const float raw = s.raw[k] + e.lp;
+                    const int new_len = s.len[k] + 1;
+                    if (slot < L.sort_cap)
+                        s.buf[slot] = Cand{raw * inv_of(s, pen_len, new_len, p.alpha), raw, k, e.token, new_len, 1};
+                };
+                lds_barrier();  // (the count is read before it grows)
+                for (int k = tid; k < K; k += kSelectThreads) {
+                    const int cnt = s.rcount[k];
+                    const float praw = s.raw[k];
+                    int n = 0;
+                    while (n < cnt && n < H && !(praw + s.sl[k * H + n].lp < tau)) ++n;
+                    if (n == 0) continue;
+                    if (n == H && cnt > H) found[atomicAdd(&st.rcount, 1)] = k;
+                    const int slot0 = atomicAdd(&st.count, n);
+                    for (int i = 0; i < n; ++i) put(slot0 + i, k, s.sl[k * H + i]);
+                }
+                lds_barrier();
+                const int nlong = st.rcount, lane = tid & 63;
+                for (int q = tid >> 6; q < nlong; q += kSelectThreads / 64) {
+                    const int k = found[q], cnt = s.rcount[k];
+                    const float praw = s.raw[k];
+                    for (int i0 = H; i0 < cnt; i0 += 64) {
+                        const bool in = i0 + lane < cnt;
+                        const ShortEntry e = list_entry(p, st, trace0 + k, in ? i0 + lane : cnt - 1);
+                        const uint64_t reach = __ballot(in && !(praw + e.lp < tau));
+                        const int n = static_cast<int>(__popcll(reach));  // a prefix: the list is sorted
+                        if (n > 0) {
+                            int slot0 = 0;
+                            if (lane == 0) slot0 = atomicAdd(&st.count, n);
+                            slot0 = __builtin_amdgcn_readfirstlane(slot0);
+                            if (lane < n) put(slot0 + lane, k, e);
+                        }
+                        if (n < 64) break;
+                    }
+                }
+                lds_barrier();
+                one_pass = st.count <= L.sort_cap;
+                if (!one_pass) {
+                    // too many: only the carried beams stay, and the lists
+                    // are offered in rounds
+                    lds_barrier();
+                    if (tid == 0) st.count = base;
+                    lds_barrier();
+                }
+            }
+        } else if (M > 0 && p.use_tau && K >= kWideBeam && forced < 0) {
             // (K <= 64 with a shortlist: lane k of wavefront 0 measures beam
             // k's prefix, eight entries a round; a lane scan places the
             // prefixes at consecutive collector slots, and the four
@@ -982,7 +1290,40 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, 
                 if (tid == 0) st.count = st.rcount;
             }
         }
-        if (M > 0 && !one_pass && forced < 0) {
+        if constexpr (WIDE) {
+            // Constrained, stepped, or too many at once: entry i of every list
+            // in turn, best first, until no list's entry could be admitted
+            // (a list is sorted, so neither could its later ones; penalties
+            // only lower a candidate).
+            if (M > 0 && !one_pass && forced < 0) {
+                const float tau = st.tau;
+                for (int i = 0; i < M; ++i) {
+                    if (tid == 0) st.overflow = 0;
+                    lds_barrier();
+                    for (int k0 = 0; k0 < K; k0 += kSelectThreads) {
+                        const int k = k0 + tid;
+                        if (k < K && i < s.rcount[k]) {
+                            const int64_t row = p.step_mode ? static_cast<int64_t>(b) * K + k : trace0 + k;
+                            const ShortEntry e = list_entry(p, st, row, i);
+                            const float praw = s.raw[k];
+                            const int new_len = s.len[k] + 1;
+                            const float inv = inv_of(s, pen_len, new_len, p.alpha);
+                            const float raw0 = praw + e.lp;
+                            if (!(raw0 < tau) && !before(st.thr, Cand{raw0 * inv, raw0, k, e.token, new_len, 1})) {
+                                st.overflow = 1;
+                                const PrefixView pre = prefix_of(p, s, b, k, cur);
+                                Cand c;
+                                if (make_cand(p, s, pre, k, praw, inv, e.token, new_len, e.lp, c)) offer(s, st, c);
+                            }
+                        }
+                        end_round(s, st, KP, L.sort_cap);
+                    }
+                    const int go = st.overflow;
+                    lds_barrier();
+                    if (go == 0) break;
+                }
+            }
+        } else if (M > 0 && !one_pass && forced < 0) {
             const float tau = st.tau;
             for (int base = 0; base < K * M; base += kSelectThreads) {
                 const int item = base + tid;
@@ -1029,8 +1370,14 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, 
         }
         lds_barrier();
         if (st.any_fail) {
+            // (64 beams at a time: each wavefront finds the same failed rows)
+            uint64_t failed = 0;
             for (int k = 0; k < K; ++k) {
-                if (s.rcount[k] != -3) continue;
+                if ((k & 63) == 0) {
+                    const int kl = k + (tid & 63);
+                    failed = __ballot(kl < K && s.rcount[kl < K ? kl : 0] == -3);
+                }
+                if (((failed >> (k & 63)) & 1ull) == 0) continue;
                 if (tid == 0) atomicAdd(&g_rescanned_rows, 1ull);
                 // drop the row's shortlisted candidates, then offer the whole row
                 for (int i = tid; i < st.count; i += kSelectThreads)
@@ -1044,6 +1391,13 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, 
                                        inv_of(s, pen_len, new_len, p.alpha), new_len, pre, L.sort_cap, KP);
             }
             compact(s, st, KP);
+        }
+
+        if constexpr (WIDE) {
+            if (coherent && st.gave_up) {  // an entry never came
+                pad_step(trace0);
+                continue;
+            }
         }
 
         // Selection (reference src/decoder.cpp:314-350): the example's best Kb.
@@ -1184,15 +1538,6 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, 
 // each worth at least lp - log(rep).
 // The kept set is the best Kb of the same candidates under the same total
 // order as the workgroup pass, so the trace is the same bit for bit.
-constexpr int kNarrowMaxK = 16;       // the running list lives in one 16-lane DPP row
-constexpr int kNarrowPf = 4;          // 16-byte prefetch registers per lane (K * M <= 512)
-constexpr int kNarrowPenCap = 1024;   // lengths with a penalty in LDS (larger ones are computed)
-constexpr int kNarrowRescanUnroll = 16;
-constexpr int kNarrowTagLoads = 4;    // tagged shortlist loads per lane in flight (overlapped decode)
-constexpr int kNarrowWaves = 4;       // examples (wavefronts) per workgroup, at most: one workgroup per CU
-constexpr int kXcds = 8;              // MI355X: 8 XCDs of 32 CUs
-constexpr int kNarrowWaveLds = 24576; // LDS per wavefront, at most (else the workgroup pass)
-
 // Lane j's candidate, wave-uniform.
 __device__ __forceinline__ Cand lane_cand(const Cand& c, int j) {
     Cand r;
@@ -1873,7 +2218,7 @@ __global__ __launch_bounds__(64 * kNarrowWaves) void select_narrow_kernel(Decode
 #pragma unroll
                         for (int u = 0; u < kNarrowRescanUnroll; ++u) {
                             const int v = v0 + 64 * u + lane;
-                            xs[u] = v < V ? load_one<DT>(base, v) : -kInf;
+                            xs[u] = load_one<DT>(base, v < V ? v : V - 1);
                         }
 #pragma unroll
                         for (int u = 0; u < kNarrowRescanUnroll; ++u) {
@@ -2006,60 +2351,16 @@ __global__ __launch_bounds__(64 * kNarrowWaves) void select_narrow_kernel(Decode
     if (lane == 0 && p.first_invalid) p.first_invalid[b] = first_bad == 0x7fffffff ? -1 : first_bad;
 }
 
-// The prefetch needs the row pass finished before the select pass starts (not
-// the overlapped decode, whose rows land while it runs) and a step's
-// shortlists within the prefetch registers, as 16-byte pairs of entries.
-bool prefetch_fits(const DecodeParams& p) {
-    return p.step_done == nullptr && !p.step_mode && p.M > 0 && (p.M & 1) == 0 && p.K <= kSelectThreads &&
-           p.K * p.M <= 2 * kPfRegs * kSelectThreads;
-}
-
-template <int DT, bool LOGITS, bool PF, bool HOLD = false>
+template <int DT, bool LOGITS, bool PF, bool HOLD = false, bool WIDE = false>
 hipError_t launch_select_variant(const DecodeParams& p, const SelectLayout& L, hipStream_t stream) {
     if (L.smem > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&select_kernel<DT, LOGITS, PF, HOLD>),
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&select_kernel<DT, LOGITS, PF, HOLD, WIDE>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(L.smem));
         if (e != hipSuccess) return e;
     }
     KernelTimer timer(kKindSelect, stream);
-    hipLaunchKernelGGL((select_kernel<DT, LOGITS, PF, HOLD>), dim3(p.B), dim3(kSelectThreads), L.smem, stream, p, L);
+    hipLaunchKernelGGL((select_kernel<DT, LOGITS, PF, HOLD, WIDE>), dim3(p.B), dim3(kSelectThreads), L.smem, stream, p, L);
     return hipGetLastError();
-}
-
-// Workgroups of the narrow pass: a multiple of kXcds (workgroups are dealt
-// to the XCDs in turn, and a persistent row pass of CUs - groups workgroups
-// leaves groups / kXcds CUs free on each), up to kNarrowWaves examples each.
-int narrow_groups(int B) { return kXcds * ((B + kXcds * kNarrowWaves - 1) / (kXcds * kNarrowWaves)); }
-int narrow_per_group(int B) {
-    const int g = narrow_groups(B);
-    return (B + g - 1) / g;
-}
-
-int narrow_pen_len(const DecodeParams& p) { return p.T + 2 < kNarrowPenCap ? p.T + 2 : kNarrowPenCap; }
-
-// One wavefront's LDS: rank keys, shortlists, candidates, penalty tables;
-// with constraints also signatures of W words per beam, prefixes, n-gram
-// lists and per-beam state (the kernel's layout).
-size_t narrow_wave_bytes(const DecodeParams& p, int W) {
-    const size_t K = static_cast<size_t>(p.K), P = static_cast<size_t>(p.prefix_cap);
-    size_t n = 1024 + sizeof(ShortEntry) * K * static_cast<size_t>(p.M) + sizeof(Cand) * 64 +
-               2 * sizeof(float) * static_cast<size_t>(narrow_pen_len(p));
-    n = (n + 15) & ~static_cast<size_t>(15);
-    if (p.constrained) {
-        const size_t P4 = (P + 3) & ~static_cast<size_t>(3);
-        n += sizeof(uint32_t) * 4 * K * static_cast<size_t>(W) + sizeof(int32_t) * (2 * K * P4 + K * P + 2 * K);
-        n = ((n + 15) & ~static_cast<size_t>(15)) + sizeof(int4) * K + sizeof(uint32_t) * K;
-    }
-    return (n + 15) & ~static_cast<size_t>(15);
-}
-
-// Signature words per beam of a constrained decode (the most of 64, 32, 16
-// that fit one wavefront's LDS), else 0; 0 for an unconstrained one.
-int narrow_sig_words(const DecodeParams& p) {
-    if (!p.constrained) return 0;
-    for (int W = 64; W >= 16; W /= 2)
-        if (narrow_wave_bytes(p, W) <= static_cast<size_t>(kNarrowWaveLds)) return W;
-    return 0;
 }
 
 template <int DT, bool LOGITS, bool CON>
@@ -2102,108 +2403,37 @@ hipError_t launch_select_typed(const DecodeParams& p, const SelectLayout& L, hip
     if (select_narrow(p))
         return p.constrained ? launch_select_narrow<DT, LOGITS, true>(p, stream)
                              : launch_select_narrow<DT, LOGITS, false>(p, stream);
+    // (wide: one instantiation, which holds its CUs whether or not a row pass
+    // runs beside it)
+    if (p.K > kListBeams) return launch_select_variant<DT, LOGITS, false, true, true>(p, L, stream);
     if (p.select_hold) return launch_select_variant<DT, LOGITS, false, true>(p, L, stream);
     return prefetch_fits(p) ? launch_select_variant<DT, LOGITS, true>(p, L, stream)
                             : launch_select_variant<DT, LOGITS, false>(p, L, stream);
 }
 
+hipError_t counter(unsigned long long& symbol, int reset, unsigned long long* value) {
+    if (reset) {
+        const unsigned long long zero = 0;
+        return hipMemcpyToSymbol(HIP_SYMBOL(symbol), &zero, sizeof(zero));
+    }
+    return hipMemcpyFromSymbol(value, HIP_SYMBOL(symbol), sizeof(*value));
+}
+
 }  // namespace
 
-std::atomic<int> g_select_kind{0};
-
-bool select_narrow(const DecodeParams& p) {
-    if (g_select_kind.load(std::memory_order_relaxed) == 1) return false;
-    if (p.step_mode || p.forced || p.pool_mult > 0 || p.M <= 0 || p.K > kNarrowMaxK || p.V > (1 << 24)) return false;
-    // constrained: n-gram blocking of n >= 2 and/or a repetition penalty
-    // (n = 1 blocking would drop most of a long prefix's shortlist entries)
-    if (p.constrained) return p.ngram != 1 && narrow_sig_words(p) > 0;
-    return p.use_tau && narrow_wave_bytes(p, 0) <= static_cast<size_t>(kNarrowWaveLds);
+template <int DT>
+hipError_t launch_select_dtype(const DecodeParams& p, const SelectLayout& L, hipStream_t stream) {
+    return p.from_logits ? launch_select_typed<DT, true>(p, L, stream) : launch_select_typed<DT, false>(p, L, stream);
 }
 
-int select_reserve_cus(const DecodeParams& p) {
-    return select_narrow(p) ? narrow_groups(p.B) : p.B;
+template <int DT>
+hipError_t rescan_counter_dtype(int reset, unsigned long long* value) {
+    return counter(g_rescanned_rows, reset, value);
 }
 
-SelectLayout select_layout(int B, int T, int K, int M, bool constrained, bool step_mode, int prefix_cap, int keep) {
-    (void)B;
-    SelectLayout L{};
-    int sc = 1;
-    while (sc < (keep > K ? keep : K) + 2 * kSelectThreads) sc <<= 1;
-    L.sort_cap = sc;
-    L.pen_len = step_mode ? 0 : T + 2;
-    auto align = [](size_t x) { return (x + 15) & ~static_cast<size_t>(15); };
-    size_t off = 0;
-    L.off_buf = off;
-    off = align(off + sizeof(Cand) * static_cast<size_t>(sc));
-    L.off_rbuf = off;
-    off = align(off + sizeof(Cand) * kRescanBuf);
-    L.off_key = off;
-    off = align(off + sizeof(uint4) * 2 * kRankMax + sizeof(int32_t) * (kSelectThreads + 64 + 1));
-    L.off_f32 = off;
-    off = align(off + sizeof(float) * (3 * static_cast<size_t>(K) + 2 * static_cast<size_t>(L.pen_len)));
-    L.off_i32 = off;
-    off = align(off + sizeof(int32_t) * 10 * static_cast<size_t>(K));
-    L.off_sl = off;
-    off = align(off + sizeof(ShortEntry) * static_cast<size_t>(K) * static_cast<size_t>(K >= kWideBeam ? M + 1 : M));
-    const size_t prefix_bytes = sizeof(int32_t) * 2 * static_cast<size_t>(K) * static_cast<size_t>(prefix_cap);
-    const size_t blk_bytes = sizeof(int32_t) * static_cast<size_t>(K) * static_cast<size_t>(prefix_cap);
-    const size_t budget = 150 * 1024;
-    L.prefix_in_lds = 0;
-    L.blk_in_lds = 0;
-    if (constrained && !step_mode && off + prefix_bytes <= budget) {
-        L.prefix_in_lds = 1;
-        L.off_prefix = off;
-        off = align(off + prefix_bytes);
-    }
-    if (constrained && off + blk_bytes <= budget) {
-        L.blk_in_lds = 1;
-        L.off_blk = off;
-        off = align(off + blk_bytes);
-    }
-    L.sig_in_lds = 0;
-    L.sig_words = 0;
-    for (int words = kSigWordsMax; words >= kSigWordsMax / 4 && !L.sig_in_lds; words /= 4) {
-        const size_t sig_bytes = sizeof(uint32_t) * 2 * static_cast<size_t>(K) * words;
-        if (L.prefix_in_lds && off + sig_bytes <= budget) {
-            L.sig_in_lds = 1;
-            L.sig_words = words;
-            L.off_sig = off;
-            off = align(off + sig_bytes);
-        }
-    }
-    L.smem = off;
-    return L;
-}
-
-hipError_t launch_select(const DecodeParams& p, const SelectLayout& L, hipStream_t stream) {
-    if (p.from_logits) {
-        switch (p.dtype) {
-            case 0: return launch_select_typed<0, true>(p, L, stream);
-            case 1: return launch_select_typed<1, true>(p, L, stream);
-            default: return launch_select_typed<2, true>(p, L, stream);
-        }
-    }
-    switch (p.dtype) {
-        case 0: return launch_select_typed<0, false>(p, L, stream);
-        case 1: return launch_select_typed<1, false>(p, L, stream);
-        default: return launch_select_typed<2, false>(p, L, stream);
-    }
-}
-
-hipError_t wait_timeout_counter(int reset, unsigned long long* value) {
-    if (reset) {
-        const unsigned long long zero = 0;
-        return hipMemcpyToSymbol(HIP_SYMBOL(g_wait_timeouts), &zero, sizeof(zero));
-    }
-    return hipMemcpyFromSymbol(value, HIP_SYMBOL(g_wait_timeouts), sizeof(*value));
-}
-
-hipError_t rescan_counter(int reset, unsigned long long* value) {
-    if (reset) {
-        const unsigned long long zero = 0;
-        return hipMemcpyToSymbol(HIP_SYMBOL(g_rescanned_rows), &zero, sizeof(zero));
-    }
-    return hipMemcpyFromSymbol(value, HIP_SYMBOL(g_rescanned_rows), sizeof(*value));
+template <int DT>
+hipError_t wait_timeout_counter_dtype(int reset, unsigned long long* value) {
+    return counter(g_wait_timeouts, reset, value);
 }
 
 }  // namespace dbs_hip
