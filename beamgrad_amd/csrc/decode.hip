@@ -264,12 +264,17 @@ hipError_t aux_for(int device, hipStream_t caller, Aux*& out) {
 // Bound of one select-pass wait: 2 s of the 100 MHz real-time counter. Test
 // knob DBS_HIP_TEST_WAIT_GIVE_UP=1: every wait needs one row more than the
 // row pass ever counts and gives up after 10 us, so the error path runs with
-// every kernel exiting normally.
+// every kernel exiting normally (the automatic choice then overlaps whatever
+// it can).
+bool wait_give_up_knob() {
+    const char* env = std::getenv("DBS_HIP_TEST_WAIT_GIVE_UP");
+    return env && env[0] == '1';
+}
+
 void wait_policy(DecodeParams& p) {
     p.wait_ticks = 200000000ull;
     p.wait_extra = 0;
-    const char* env = std::getenv("DBS_HIP_TEST_WAIT_GIVE_UP");
-    if (env && env[0] == '1') {
+    if (wait_give_up_knob()) {
         p.wait_ticks = 1000ull;
         p.wait_extra = 1;
     }
@@ -312,7 +317,8 @@ hipError_t launch_decode(const DecodeParams& p0, const DecodeLayout& L, hipStrea
     Aux* aux = nullptr;
     const int mode = g_overlap.load(std::memory_order_relaxed);
     bool want = allow_overlap && !p.step_mode && p.T > 1 &&
-                (mode == 1 || (mode == -1 && (p.constrained || row_pass_persistent(p) || !select_narrow(p))));
+                (mode == 1 || (mode == -1 && (p.constrained || row_pass_persistent(p) || !select_narrow(p) ||
+                                              wait_give_up_knob())));
     // Under stream capture the two passes run one after the other: a graph
     // may start its branches in any order, and a select pass started before
     // the row pass would wait for rows nobody is producing.
@@ -323,8 +329,8 @@ hipError_t launch_decode(const DecodeParams& p0, const DecodeLayout& L, hipStrea
         e = aux_for(device, stream, aux);
         if (e != hipSuccess) return e;
     }
-    const int reserve = select_reserve_cus(p);
     const bool persistent = row_pass_persistent(p);
+    const int reserve = select_reserve_cus(p, persistent);
     // Beside a row pass of one workgroup per row, a select pass of at most
     // one workgroup per 8 CUs holds its CUs (select_hold: the workgroup pass,
     // and the one-wavefront pass of a constrained decode); a larger one
@@ -332,7 +338,7 @@ hipError_t launch_decode(const DecodeParams& p0, const DecodeLayout& L, hipStrea
     // when its select pass holds its CUs (shared, its steps ran ~3x slower
     // than alone).
     const bool hold = !persistent && aux && 8 * reserve <= aux->cus;
-    if (aux && mode == -1 && !p.constrained && !persistent && !hold) aux = nullptr;
+    if (aux && mode == -1 && !p.constrained && !persistent && !hold && !wait_give_up_knob()) aux = nullptr;
     // One launch zeroes the row logsumexps (rows the search does not read keep
     // 0) and, in the overlapped decode, the counters and the RowInfo and
     // shortlist words (tag 0: not written).

@@ -208,6 +208,9 @@ bool row_relay_eligible(const DecodeParams& p);
 // its full register capacity, so shorter rows take the resident pass).
 bool row_relay_preferred(const DecodeParams& p);
 hipError_t launch_row_relay(const DecodeParams& p, int64_t rows, hipStream_t stream);
+// Logits rows of any size and alignment, read twice (row_stream.hip).
+bool row_stream_eligible(const DecodeParams& p);
+hipError_t launch_row_stream(const DecodeParams& p, int64_t rows, hipStream_t stream);
 bool row_logprob_eligible(const DecodeParams& p);
 hipError_t launch_row_logprob(const DecodeParams& p, int64_t rows, hipStream_t stream);
 extern std::atomic<int> g_row_pass_kind;  // dbs_hip_set_row_pass
@@ -225,8 +228,9 @@ hipError_t wait_timeout_counter_dtype(int reset, unsigned long long* value);
 // (g_select_kind 1) keeps the workgroup pass.
 bool select_narrow(const DecodeParams& p);
 extern std::atomic<int> g_select_kind;
-// CUs the overlapped decode leaves free for the select pass.
-int select_reserve_cus(const DecodeParams& p);
+// CUs the overlapped decode leaves free for the select pass, beside a
+// persistent row pass (one workgroup per CU) or one of several per CU.
+int select_reserve_cus(const DecodeParams& p, bool persistent);
 
 // Rows the select pass rescanned in full (reset = 1 clears the count).
 hipError_t rescan_counter(int reset, unsigned long long* value);

@@ -22,8 +22,9 @@ bool select_narrow(const DecodeParams& p) {
     return p.use_tau && narrow_wave_bytes(p, 0) <= static_cast<size_t>(kNarrowWaveLds);
 }
 
-int select_reserve_cus(const DecodeParams& p) {
-    return select_narrow(p) ? narrow_groups(p.B) : p.B;
+int select_reserve_cus(const DecodeParams& p, bool persistent) {
+    if (!select_narrow(p)) return p.B;
+    return persistent ? narrow_groups(p.B) : (p.B + kNarrowWaves - 1) / kNarrowWaves;
 }
 
 SelectLayout select_layout(int B, int T, int K, int M, bool constrained, bool step_mode, int prefix_cap, int keep) {

@@ -1611,13 +1611,226 @@ __device__ __forceinline__ void issue_tagged(const DecodeParams& p, int b, int t
     }
 }
 
-// HOLD: as the workgroup pass's (every register of its SIMDs claimed, so
-// no row-pass wavefront joins a CU that holds one of its workgroups).
-template <int DT, bool LOGITS, bool PF, bool CON, bool HOLD = false>
-__global__ __launch_bounds__(64 * kNarrowWaves) void select_narrow_kernel(DecodeParams p, int pen_len, int wave_bytes,
-                                                                         int sig_words) {
-    if constexpr (HOLD) asm volatile("" ::: "a255");
-    extern __shared__ __align__(16) unsigned char smem_all[];
+// The steps of an unconstrained decode of at most kGridBeams beams, the
+// candidates in a grid: lane (k, j) = k K + j holds entry j of beam k's
+// shortlist (only the first K of a list can be selected), and every lane of
+// beam k its state, so that a step moves nothing between lanes but the
+// candidates' keys and the selection, through LDS:
+//   * the lane's entry and its row's RowInfo, loaded kGridAhead steps ahead
+//     (three words; a step's chain is shorter than a load's latency);
+//   * tau, the largest K-th entry's raw: candidates below it are not selected;
+//   * the keys of the others, packed in LDS, and each one's rank among them:
+//     (raw, parent, token) where every beam is expanded (one length: the score
+//     is a nondecreasing function of raw), else (score, raw, parent, token);
+//   * the selection, by rank, back into every lane of its beam.
+// Loads, and stores through views that drop the lanes that have none, are
+// never under a branch, so that a wait for a step's words is a wait for the
+// operations before them and leaves the later steps' in flight. Bound by the
+// chain of LDS round trips and lane operations, 1.3 us a step: 8 x 32 x 4 x
+// 32000 f32 42 us (the general step, 3.1 us: 97).
+// Returns the first step not taken: steps_b, or a step whose rows need a
+// full read or whose words never came (gave_up). s: 64 keys of 16 bytes, then
+// the selection (kGridBeams of 16 bytes, over the shortlists).
+struct GridState {
+    float raw;
+    int len, last, ended;
+};
+
+struct GridWords {
+    uint32_t lp, tok;         // the entry (its tag in tok in the overlapped decode)
+    uint32_t i0, i1, i2, i3;  // the row's RowInfo (tags in i1 and i3)
+};
+
+template <bool LOGITS>
+__device__ __forceinline__ int grid_steps(const DecodeParams& p, int b, int t, int steps_b, int Kb, int eos_b,
+                                          GridState& g, uint4* s_key, const float* s_pen, const float* s_inv,
+                                          int pen_len, int lane, bool& any_invalid, int& first_bad, bool& gave_up) {
+    const int K = p.K, T = p.T, M = p.M;
+    const int k = lane / K, j = lane - k * K;
+    const bool on = k < K;  // (K * K lanes of the grid)
+    const int kc = on ? k : 0, jc = on ? j : 0;
+    const bool coherent = p.step_done != nullptr;
+    uint2* const s_key2 = reinterpret_cast<uint2*>(s_key);
+    uint4* const s_sel = s_key + 64;
+    const bool head = on && j == 0;
+    // trace views of this example: lanes with nothing to store use an offset
+    // past their end
+    const int64_t ex = static_cast<int64_t>(b) * T * K;
+    const int trace_bytes = 4 * T * K;
+    auto view = [&](void* base, int esz) {
+        return __builtin_amdgcn_make_buffer_rsrc(static_cast<char*>(base) + ex * esz, 0, base ? trace_bytes / 4 * esz : 0,
+                                                 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t v_tok = view(p.tokens, 4), v_par = view(p.parents, 4), v_len = view(p.lengths, 4),
+                                 v_score = view(p.scores, 4), v_raw = view(p.raw_scores, 4),
+                                 v_flp = view(p.from_logprob, 1), v_lse = view(LOGITS ? p.row_lse : nullptr, 4);
+
+    GridWords ring[kGridAhead];
+    auto issue = [&](GridWords& w, int tn) __attribute__((always_inline)) {
+        const int64_t row = ex + static_cast<int64_t>(tn < steps_b ? tn : steps_b - 1) * K + kc;
+        const uint32_t* e = reinterpret_cast<const uint32_t*>(p.shortlist + row * M + jc);
+        const uint32_t* r = reinterpret_cast<const uint32_t*>(p.rowinfo + row);
+        if (coherent) {
+            (void)read_tagged(e, w.lp, w.tok);
+            (void)read_tagged(r, w.i0, w.i1);
+            (void)read_tagged(r + 2, w.i2, w.i3);
+        } else {
+            const uint2 ev = *reinterpret_cast<const uint2*>(e);
+            const uint4 iv = *reinterpret_cast<const uint4*>(r);
+            w.lp = ev.x;
+            w.tok = ev.y;
+            w.i0 = iv.x;
+            w.i1 = iv.y;
+            w.i2 = iv.z;
+            w.i3 = iv.w;
+        }
+    };
+    // One step from words w; false: not taken (the state is as before it).
+    auto step = [&](GridWords& w, int tt) __attribute__((always_inline)) -> bool {
+        const bool live = on && g.raw < kInf && g.raw > -kInf;
+        const bool carried = live && eos_b >= 0 && g.ended != 0;
+        const bool read = live && !carried;
+        uint32_t lpw = w.lp, tokw = w.tok, i0 = w.i0, i1 = w.i1, i2 = w.i2, i3 = w.i3;
+        issue(w, tt + kGridAhead);
+        if (coherent) {
+            // words not yet written (tag 0) are waited for
+            const bool miss_info = read && (i1 == 0u || i3 == 0u);
+            if (__builtin_amdgcn_ballot_w64(miss_info || (read && tokw == 0u)) != 0) {
+                const int64_t row = ex + static_cast<int64_t>(tt) * K + kc;
+                const uint32_t* e = reinterpret_cast<const uint32_t*>(p.shortlist + row * M + jc);
+                const uint32_t* r = reinterpret_cast<const uint32_t*>(p.rowinfo + row);
+                bool ok = true;
+                if (read) {
+                    if (i1 == 0u) ok = wait_tagged(p, r, i0, i1);
+                    if (ok && i3 == 0u) ok = wait_tagged(p, r + 2, i2, i3);
+                    if (ok && tokw == 0u && jc < static_cast<int>(i1) - 2) ok = wait_tagged(p, e, lpw, tokw);
+                }
+                if (__builtin_amdgcn_ballot_w64(!ok) != 0) {
+                    gave_up = true;
+                    return false;
+                }
+            }
+            i1 -= 2u;
+            i3 -= 1u;
+            tokw -= 1u;
+        }
+        const int cnt = static_cast<int>(i1);
+        const float lse = bits_f32(i0), bound = bits_f32(i2);
+        const uint64_t bad_m = __builtin_amdgcn_ballot_w64(read && i3 != 0u);
+        const float inv = (tt + 1 < pen_len) ? s_inv[tt + 1] : 1.0f / length_penalty(tt + 1, p.alpha);
+        // the lane's candidate
+        float raw = g.raw + bits_f32(lpw);
+        float score = raw * inv;
+        int token = static_cast<int>(tokw);
+        bool have = read && j < cnt;
+        const float tau = wave_max_dpp(have && j == K - 1 ? raw : -kInf);
+        have = have && !(raw < tau);
+        const uint64_t carried_m = __builtin_amdgcn_ballot_w64(carried);
+        if (carried_m != 0) {
+            const int l = g.len > 1 ? g.len : 1;
+            const float pen = l < pen_len ? s_pen[l] : length_penalty(l, p.alpha);
+            if (carried && j == 0) {
+                raw = g.raw;
+                score = g.raw / pen;
+                token = is_eos_of(p, b, g.last) ? g.last : eos_b;
+                have = true;
+            }
+        }
+        have = have && (score > -kInf || raw > -kInf);  // ranks before the dead sentinel
+        const uint64_t m = __builtin_amdgcn_ballot_w64(have);
+        const int n = static_cast<int>(__popcll(m));
+        const int before_me = static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
+                                                                         __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u)));
+        const int pos = have ? before_me : n + (lane - before_me);  // the others: zero keys after them
+        const uint32_t low = (static_cast<uint32_t>(k) << 24) | (static_cast<uint32_t>(token) & 0xffffffu);
+        const uint32_t k0 = have ? 0xffffffffu - low : 0u, k1 = have ? ordered_key(raw) : 0u;
+        int rank = 0;
+        if (carried_m == 0) {
+            s_key2[pos] = make_uint2(k0, k1);
+            wave_sync();
+            for (int q = 0; q < n; q += 8) {  // (64 keys: the last round stays within them)
+                uint4 x[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) x[u] = s_key[q / 2 + u];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    count_above64(rank, k0, k1, x[u].x, x[u].y);
+                    count_above64(rank, k0, k1, x[u].z, x[u].w);
+                }
+            }
+        } else {
+            const uint32_t k2 = have ? ordered_key(score) : 0u;
+            s_key[pos] = make_uint4(k0, k1, k2, 0u);
+            wave_sync();
+            for (int q = 0; q < n; q += 4) {
+                uint4 x[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) x[u] = s_key[q + u];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) count_above96(rank, k0, k1, k2, x[u].x, x[u].y, x[u].z);
+            }
+        }
+        const int nsel = n < Kb ? n : Kb;
+        const uint32_t meta = static_cast<uint32_t>(carried ? (g.len > 1 ? g.len : 1) : tt + 1) |
+                              (carried ? 0u : 0x40000000u) | (g.ended != 0 ? 0x80000000u : 0u);
+        if (have && rank < Kb) s_sel[rank] = make_uint4(f32_bits(score), f32_bits(raw), low, meta);
+        wave_sync();
+        const uint4 mine = s_sel[kc];
+        const uint4 kth = s_sel[Kb - 1];
+        // Exactness: every candidate left out of a row's list (its entries
+        // from K on too: K others of the row come first) has raw <= fl(p +
+        // bound); the row passes when the Kb-th selected candidate ranks
+        // strictly before that bound's score and raw.
+        bool fail = read && cnt < 0;
+        if (read && bound > -kInf) {
+            const float X = g.raw + bound;
+            const float SX = X * inv;
+            const float ks = nsel >= Kb ? bits_f32(kth.x) : -kInf, kr = nsel >= Kb ? bits_f32(kth.y) : -kInf;
+            fail = fail || (X > -kInf && !((ks > SX) || (ks == SX && kr > X)));
+        }
+        if (__builtin_amdgcn_ballot_w64(fail) != 0) return false;
+        if (bad_m != 0) {
+            any_invalid = true;
+            const int at = tt * K + (__ffsll(static_cast<long long>(bad_m)) - 1) / K;  // steps in order, beams in order
+            first_bad = at < first_bad ? at : first_bad;
+        }
+        const bool sel = on && k < nsel;
+        const int parent = sel ? static_cast<int>(mine.z >> 24) : -1;
+        const int tok = sel ? static_cast<int>(mine.z & 0xffffffu) : -1;
+        const int length = sel ? static_cast<int>(mine.w & 0x3fffffffu) : 0;
+        const float sc = sel ? bits_f32(mine.x) : -kInf, rw = sel ? bits_f32(mine.y) : -kInf;
+        const int flp = sel ? static_cast<int>((mine.w >> 30) & 1u) : 0;
+        const int at = head ? (tt * K + k) * 4 : trace_bytes;
+        __builtin_amdgcn_raw_buffer_store_b32(static_cast<uint32_t>(tok), v_tok, at, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(static_cast<uint32_t>(parent), v_par, at, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(static_cast<uint32_t>(length), v_len, at, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(f32_bits(sc), v_score, at, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(f32_bits(rw), v_raw, at, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b8(static_cast<uint8_t>(flp), v_flp, at / 4, 0, 0);
+        if constexpr (LOGITS)
+            __builtin_amdgcn_raw_buffer_store_b32(f32_bits(lse), v_lse, read ? at : trace_bytes, 0, 0);
+        g.raw = rw;
+        g.len = length;
+        g.last = tok;
+        g.ended = sel && ((mine.w >> 31) != 0u || is_eos_of(p, b, tok)) ? 1 : 0;
+        wave_sync();  // the keys' and the selection's LDS may be reused
+        return true;
+    };
+#pragma unroll
+    for (int u = 0; u < kGridAhead; ++u) issue(ring[u], t + u);
+    for (;;) {
+#pragma unroll
+        for (int u = 0; u < kGridAhead; ++u) {
+            if (t >= steps_b) return t;
+            if (!step(ring[u], t)) return t;
+            ++t;
+        }
+    }
+}
+
+template <int DT, bool LOGITS, bool PF, bool CON>
+__device__ __forceinline__ void narrow_example(const DecodeParams& p, int pen_len, int wave_bytes, int sig_words,
+                                               unsigned char* smem_all) {
     const int K = p.K, T = p.T, M = p.M, V = p.V;
     // up to kNarrowWaves examples per workgroup, one per wavefront, each with
     // its own LDS; the wavefronts never wait for each other
@@ -1695,8 +1908,13 @@ __global__ __launch_bounds__(64 * kNarrowWaves) void select_narrow_kernel(Decode
         if (lane + 192 < n4) pf3 = src4[lane + 192];
     };
     bool have_pf = false;
+    // Unconstrained decodes of at most kGridBeams beams: their steps go
+    // through grid_steps below, and only those that fail its exactness check
+    // (and the padding steps) through the general step. (The test knob for
+    // waits that give up forces the general step's counted wait.)
+    const bool grid = !CON && K <= kGridBeams && M >= K && p.wait_extra == 0;
     if constexpr (PF) {
-        have_pf = steps_b > 0;
+        have_pf = steps_b > 0 && !grid;
         if (have_pf) prefetch(0);
     }
     // A step's trace is stored during the next step and its row logsumexps
@@ -1751,9 +1969,25 @@ __global__ __launch_bounds__(64 * kNarrowWaves) void select_narrow_kernel(Decode
     // before, and the tail joins the signature when the beam grows.
     uint32_t tail_h = 0u;
     bool tail_v = false;
+    const int gk = lane / K < K ? lane / K : 0;  // the beam of this lane in grid_steps
     wave_sync();
 
     for (int t = 0; t < T; ++t) {
+        if constexpr (!CON) {
+            if (grid && t < steps_b && !gave_up) {
+                GridState g{__shfl(raw, gk), __shfl(len, gk), __shfl(last, gk), __shfl(ended ? 1 : 0, gk)};
+                t = grid_steps<LOGITS>(p, b, t, steps_b, Kb, eos_b, g, s_key, s_pen, s_inv, pen_len, lane, any_invalid,
+                                       first_bad, gave_up);
+                const int src = lane < K ? lane * K : 0;
+                const float raw_k = __shfl(g.raw, src);  // (every lane shuffles)
+                const int ended_k = __shfl(g.ended, src);
+                len = __shfl(g.len, src);
+                last = __shfl(g.last, src);
+                raw = beam ? raw_k : -kInf;
+                ended = beam && ended_k != 0;
+                if (t >= T) break;
+            }
+        }
         const int64_t trace0 = (static_cast<int64_t>(b) * T + t) * K;
         bool pad = t >= steps_b || gave_up;
         const bool live = beam && raw < kInf && raw > -kInf;
@@ -1920,10 +2154,10 @@ __global__ __launch_bounds__(64 * kNarrowWaves) void select_narrow_kernel(Decode
         // the pending stores (after the loads, so that waiting for the loads
         // never waits for them)
         if constexpr (PF) {
-            have_pf = t + 1 < steps_b;
+            have_pf = t + 1 < steps_b && !grid;
             if (have_pf) prefetch(t + 1);
         }
-        if (coherent && t + 1 < steps_b) {
+        if (coherent && t + 1 < steps_b && !grid) {
             issue_tagged(p, b, t + 1, lane, tw);
             spec = true;
         }
@@ -2329,6 +2563,7 @@ __global__ __launch_bounds__(64 * kNarrowWaves) void select_narrow_kernel(Decode
         len = c.length;
         last = c.token;
         wave_sync();
+        if (grid) flush();
     }
     flush();
 
@@ -2349,6 +2584,21 @@ __global__ __launch_bounds__(64 * kNarrowWaves) void select_narrow_kernel(Decode
     // example did not complete (an overlapped wait gave up)
     if (lane == 0 && p.invalid) p.invalid[b] = static_cast<uint8_t>(gave_up ? 2 : (any_invalid ? 1 : 0));
     if (lane == 0 && p.first_invalid) p.first_invalid[b] = first_bad == 0x7fffffff ? -1 : first_bad;
+}
+
+// HOLD: as the workgroup pass's (every register of its SIMDs claimed, so no
+// row-pass wavefront joins a CU that holds one of its workgroups): its
+// workgroups have kNarrowWaves wavefronts, one per SIMD, and those without an
+// example, or done with it, wait at the end for the others. (With fewer
+// wavefronts the row pass shared the CU, and 16 examples beside a row pass of
+// f32 rows made next to no step until it had ended.)
+template <int DT, bool LOGITS, bool PF, bool CON, bool HOLD = false>
+__global__ __launch_bounds__(64 * kNarrowWaves) void select_narrow_kernel(DecodeParams p, int pen_len, int wave_bytes,
+                                                                         int sig_words) {
+    if constexpr (HOLD) asm volatile("" ::: "a255");
+    extern __shared__ __align__(16) unsigned char smem_all[];
+    narrow_example<DT, LOGITS, PF, CON>(p, pen_len, wave_bytes, sig_words, smem_all);
+    if constexpr (HOLD) __syncthreads();
 }
 
 template <int DT, bool LOGITS, bool PF, bool HOLD = false, bool WIDE = false>
@@ -2372,22 +2622,22 @@ hipError_t launch_select_narrow(const DecodeParams& p, hipStream_t stream) {
     // 16-byte pairs of entries within the prefetch registers
     const bool pf = p.step_done == nullptr && (p.M & 1) == 0 && p.K * p.M <= 2 * 64 * kNarrowPf;
     KernelTimer timer(kKindSelect, stream);
-    const int per = narrow_per_group(p.B);
+    const int per = p.select_hold ? kNarrowWaves : narrow_per_group(p.B);
     const dim3 grid((p.B + per - 1) / per), block(64 * per);
     const size_t smem = static_cast<size_t>(wave_bytes) * per;
     if (smem > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(pf ? &select_narrow_kernel<DT, LOGITS, true, CON>
                                                                            : &select_narrow_kernel<DT, LOGITS, false, CON>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
-        if (e == hipSuccess && CON)
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(&select_narrow_kernel<DT, LOGITS, false, true, true>),
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute(reinterpret_cast<const void*>(&select_narrow_kernel<DT, LOGITS, false, CON, true>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
         if (e != hipSuccess) return e;
     }
-    // beside a row pass of one workgroup per row: constrained decodes hold
-    // their CUs (p.select_hold)
-    if (CON && p.select_hold)
-        hipLaunchKernelGGL((select_narrow_kernel<DT, LOGITS, false, true, true>), grid, block, smem, stream, p, pen_len,
+    // beside a row pass of several workgroups per CU it holds its CUs
+    // (p.select_hold)
+    if (p.select_hold)
+        hipLaunchKernelGGL((select_narrow_kernel<DT, LOGITS, false, CON, true>), grid, block, smem, stream, p, pen_len,
                            wave_bytes, W);
     else if (pf)
         hipLaunchKernelGGL((select_narrow_kernel<DT, LOGITS, true, CON>), grid, block, smem, stream, p, pen_len,

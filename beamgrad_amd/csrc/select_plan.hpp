@@ -29,6 +29,8 @@ constexpr int kWideRank = 4;  // candidates per thread of the rank compaction be
 
 // The narrow select pass (select_kernels.hpp).
 constexpr int kNarrowMaxK = 16;       // the running list lives in one 16-lane DPP row
+constexpr int kGridBeams = 8;         // beams whose K * K candidates fit one wavefront's lanes (grid_steps)
+constexpr int kGridAhead = 4;         // steps its words are loaded ahead
 constexpr int kNarrowPf = 4;          // 16-byte prefetch registers per lane (K * M <= 512)
 constexpr int kNarrowPenCap = 1024;   // lengths with a penalty in LDS (larger ones are computed)
 constexpr int kNarrowRescanUnroll = 16;
