@@ -330,13 +330,10 @@ constexpr int kRankSurvivors = 128;  // up to this many survivors are placed by 
 // One wavefront: orders the n row survivors (finite x >= theta) kept in LDS
 // and writes the row's shortlist (the best M allowed tokens by value desc,
 // token asc, as log-probs) and RowInfo: the bound on every allowed token left
-// out is the (M+1)-th allowed survivor, else theta. FILTER: the survivors may
-// include statically masked tokens (banned, EOS below min_length of example
-// b), which are dropped here (key 0 sorts last).
-template <bool LOGITS, bool FILTER>
+// out is the (M+1)-th survivor, else theta.
+template <bool LOGITS>
 __device__ void finish_row_wave(const DecodeParams& p, int64_t r, float lse, float theta, bool any_bad,
-                                uint64_t* s_key, float* s_x, int n, int lane, int b, bool mask_eos,
-                                bool signal = true) {
+                                uint64_t* s_key, float* s_x, int n, int lane) {
     const int M = p.M;
     const bool coherent = p.step_done != nullptr;
     RowInfo info;
@@ -350,45 +347,30 @@ __device__ void finish_row_wave(const DecodeParams& p, int64_t r, float lse, flo
         } else {
             int np = 1;
             while (np < n) np <<= 1;
-            int dropped = 0;
-            if constexpr (FILTER) {
-                for (int i0 = 0; i0 < n; i0 += 64) {
-                    const int i = i0 + lane;
-                    bool drop = false;
-                    if (i < n) {
-                        const int v = static_cast<int>(0xffffffffu - static_cast<uint32_t>(s_key[i] & 0xffffffffu));
-                        drop = static_masked(p, b, v, mask_eos);
-                        if (drop) s_key[i] = 0;
-                    }
-                    dropped += __popcll(__ballot(drop));
-                }
-            }
-            n -= dropped;
             const int cnt = n < M ? n : M;
             ShortEntry* out = p.shortlist + r * M;
             float bx = theta;
-            if (n + dropped <= kRankSurvivors) {
+            if (n <= kRankSurvivors) {
                 // Few survivors: each lane ranks its own by counting the keys
-                // above it (keys are distinct; dropped ones are 0) and writes
-                // it in place; rank M is the bound.
-                const int nall = n + dropped;
+                // above it (keys are distinct) and writes it in place; rank M
+                // is the bound.
                 wave_sync();
                 int bound_lane = -1;
                 float bound_x = -kInf;
-                for (int i0 = 0; i0 < nall; i0 += 64) {
+                for (int i0 = 0; i0 < n; i0 += 64) {
                     const int i = i0 + lane;
-                    const uint64_t ki = i < nall ? s_key[i] : 0;
+                    const uint64_t ki = i < n ? s_key[i] : 0;
                     int rank = 0;
                     int jj = 0;
-                    for (; jj + 8 <= nall; jj += 8) {  // eight keys in flight
+                    for (; jj + 8 <= n; jj += 8) {  // eight keys in flight
                         uint64_t kk[8];
 #pragma unroll
                         for (int u = 0; u < 8; ++u) kk[u] = s_key[jj + u];
 #pragma unroll
                         for (int u = 0; u < 8; ++u) rank += static_cast<int>(kk[u] > ki);
                     }
-                    for (; jj < nall; ++jj) rank += static_cast<int>(s_key[jj] > ki);
-                    const bool live = i < nall && ki != 0;
+                    for (; jj < n; ++jj) rank += static_cast<int>(s_key[jj] > ki);
+                    const bool live = i < n && ki != 0;
                     const float x = live ? s_x[i] : 0.0f;
                     if (live && rank < M) {
                         const int32_t tok = static_cast<int32_t>(0xffffffffu - static_cast<uint32_t>(ki & 0xffffffffu));
@@ -402,7 +384,7 @@ __device__ void finish_row_wave(const DecodeParams& p, int64_t r, float lse, flo
                 }
                 if (n > M) bx = bound_x;
             } else {
-                for (int i = n + dropped + lane; i < np; i += 64) s_key[i] = 0;
+                for (int i = n + lane; i < np; i += 64) s_key[i] = 0;
                 wave_sync();
                 for (int kk = 2; kk <= np; kk <<= 1) {
                     for (int jj = kk >> 1; jj > 0; jj >>= 1) {
@@ -435,7 +417,7 @@ __device__ void finish_row_wave(const DecodeParams& p, int64_t r, float lse, flo
         }
     }
     if (lane == 0) publish_rowinfo(p.rowinfo + r, info, coherent);
-    if (signal) signal_row_done(p, r, lane);  // else the caller signals later
+    signal_row_done(p, r, lane);
 }
 
 }  // namespace dbs_hip

@@ -194,27 +194,21 @@ hipError_t launch_decode(const DecodeParams& p, const DecodeLayout& L, hipStream
 size_t sync_bytes(int B, int T);           // overlapped-decode counters in the workspace
 extern std::atomic<int> g_overlap;         // dbs_hip_set_decode_overlap
 hipError_t launch_row_pass(const DecodeParams& p, hipStream_t stream);
-// Whether launch_row_pass would run one of the persistent (one workgroup per
-// CU) row passes for p.
+// Whether launch_row_pass would run the row pass of one persistent workgroup
+// per CU (the relay) for p.
 bool row_pass_persistent(const DecodeParams& p);
-// Row pass that keeps each row on chip (16-bit rows, V % 8 == 0, 16-byte
-// aligned, V <= 155648); launch_row_pass uses it when eligible.
-bool row_resident_eligible(const DecodeParams& p);
-hipError_t launch_row_resident(const DecodeParams& p, int64_t rows, hipStream_t stream);
-bool row_pipe_eligible(const DecodeParams& p);
 // bfloat16 logits, both segments of a 512-thread workgroup relaying (row_relay.hip)
 bool row_relay_eligible(const DecodeParams& p);
 // The relay row pass is the default for the rows it fills (it always folds
-// its full register capacity, so shorter rows take the resident pass).
+// its full register capacity, so shorter rows take the stream pass).
 bool row_relay_preferred(const DecodeParams& p);
 hipError_t launch_row_relay(const DecodeParams& p, int64_t rows, hipStream_t stream);
-// Logits rows of any size and alignment, read twice (row_stream.hip).
+// Rows of any type, size and alignment, read twice (row_stream.hip).
 bool row_stream_eligible(const DecodeParams& p);
 hipError_t launch_row_stream(const DecodeParams& p, int64_t rows, hipStream_t stream);
 bool row_logprob_eligible(const DecodeParams& p);
 hipError_t launch_row_logprob(const DecodeParams& p, int64_t rows, hipStream_t stream);
 extern std::atomic<int> g_row_pass_kind;  // dbs_hip_set_row_pass
-hipError_t launch_row_pipe(const DecodeParams& p, int64_t rows, hipStream_t stream);
 hipError_t launch_select(const DecodeParams& p, const SelectLayout& L, hipStream_t stream);
 // The kernels of one input type (0 f32, 1 f16, 2 bf16), and their counters.
 template <int DT>

@@ -35,20 +35,6 @@ __device__ __forceinline__ uint32_t pk_min_u16(uint32_t a, uint32_t b) {
 __device__ __forceinline__ uint32_t pk_sub_sat_u16(uint32_t a, uint32_t b) {
     return __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(v2u16, a), __builtin_bit_cast(v2u16, b)));
 }
-__device__ __forceinline__ uint32_t pk_sub_sat_i16(uint32_t a, uint32_t b) {
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(v2i16, a), __builtin_bit_cast(v2i16, b)));
-}
-__device__ __forceinline__ uint32_t pk_add_u16(uint32_t a, uint32_t b) {  // wrapping
-    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2u16, a) + __builtin_bit_cast(v2u16, b));
-}
-__device__ __forceinline__ uint32_t pk_sign_fill_i16(uint32_t a) {
-    const v2i16 fifteen = {15, 15};
-    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2i16, a) >> fifteen);
-}
-__device__ __forceinline__ uint32_t pk_shl2_u16(uint32_t a) {
-    const v2u16 two = {2, 2};
-    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2u16, a) << two);
-}
 
 // Buffer view of one row (bytes [0, nbytes)): loads past its end return
 // zeros instead of touching memory.
@@ -70,12 +56,6 @@ __device__ __forceinline__ float pattern_value(uint32_t h) {
 __device__ __forceinline__ int key16(uint32_t h) {
     const int s = static_cast<int16_t>(h);
     return s < 0 ? (s ^ 0x7fff) : s;
-}
-
-// The 16-bit pattern of theta (a value of the row, or -inf).
-template <int DT>
-__device__ __forceinline__ uint32_t value_pattern(float x) {
-    return DT == 2 ? (f32_bits(x) >> 16) : f32_to_f16_rne(x);
 }
 
 // Whether the bfloat16 term table covers a row with maximum m; u_lo out.

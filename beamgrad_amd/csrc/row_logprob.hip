@@ -38,8 +38,8 @@ namespace dbs_hip {
 
 namespace {
 
-constexpr int kLpThreads = 256;
-constexpr int kLpMaxBlocks = 40;  // 16-byte blocks per thread, at most
+constexpr int kLpThreads = 256;   // or twice as many, for the longest rows
+constexpr int kLpMaxBlocks = 52;  // 16-byte blocks per thread, at most
 constexpr int kLpBlockCap = 512;  // blocks holding survivors, at most (else the row is read in full)
 
 // Element i of a block as f32. binary16 goes through the hardware conversion,
@@ -74,7 +74,7 @@ __device__ __forceinline__ void set_neg_inf(v4u32& d, int i) {
 // Not valid (no row left): the same loads through an empty buffer view, which
 // return zeros and touch no memory, so the loads never sit under a branch.
 // Blocks C0 .. C1 - 1 only (the row is loaded in two parts).
-template <int DT, int C, int C0 = 0, int C1 = C>
+template <int NT, int DT, int C, int C0 = 0, int C1 = C>
 __device__ __forceinline__ int load_row(const DecodeParams& p, int64_t r, bool valid, int tid, v4u32 (&d)[C]) {
     constexpr int esz = DT == 0 ? 4 : 2;
     const uintptr_t a0 = reinterpret_cast<uintptr_t>(p.x) + static_cast<uintptr_t>(valid ? r : 0) * p.V * esz;
@@ -83,7 +83,8 @@ __device__ __forceinline__ int load_row(const DecodeParams& p, int64_t r, bool v
     const __amdgpu_buffer_rsrc_t rs =
         __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(a0 - lead), 0, 16 * nblk, 0x00020000);
 #pragma unroll
-    for (int c = C0; c < C1; ++c) d[c] = __builtin_amdgcn_raw_buffer_load_b128(rs, 16 * tid, 4096 * c, kRowLoadPolicy);
+    for (int c = C0; c < C1; ++c)  // (the scalar offset stays within the view)
+        d[c] = __builtin_amdgcn_raw_buffer_load_b128(rs, 16 * tid, min(16 * NT * c, 16 * nblk), kRowLoadPolicy);
     return lead / esz;
 }
 
@@ -127,11 +128,11 @@ __device__ __forceinline__ void next_row_options(const DecodeParams& p, int64_t 
 // registers to the scan (three workgroups per CU at 32 blocks per thread).
 // Barriers after that point order LDS only (lds_barrier), which keeps the
 // loads outstanding across them.
-template <int DT, int C>
-__global__ __launch_bounds__(kLpThreads) __attribute__((amdgpu_waves_per_eu(C <= 32 ? 3 : 1))) void row_logprob_kernel(DecodeParams p, int64_t rows) {
+template <int DT, int C, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(C <= 32 && NT == kLpThreads ? 3 : 2))) void row_logprob_kernel(DecodeParams p, int64_t rows) {
     __shared__ uint64_t s_key[kSurvivorCap];
     __shared__ float s_x[kSurvivorCap];
-    __shared__ __align__(16) uint32_t s_tkey[kLpThreads];
+    __shared__ __align__(16) uint32_t s_tkey[NT];
     __shared__ v4u32 s_blk[kLpBlockCap];
     __shared__ int s_blk_v0[kLpBlockCap];
     __shared__ RowSlot s_slot;
@@ -169,14 +170,14 @@ __global__ __launch_bounds__(kLpThreads) __attribute__((amdgpu_waves_per_eu(C <=
     bool mask_eos = s_slot_mask_eos != 0;
     int eos_b = s_slot_eos;
     v4u32 d[C];
-    int lead_e = load_row<DT, C>(p, r, r < rows, tid, d);
+    int lead_e = load_row<NT, DT, C>(p, r, r < rows, tid, d);
 
     while (r < rows) {
 
         // Elements outside the row become -inf.
 #pragma unroll
         for (int c = 0; c < C; ++c) {
-            const int v0 = (c * kLpThreads + tid) * epb - lead_e;
+            const int v0 = (c * NT + tid) * epb - lead_e;
             if (v0 < 0 || v0 + epb > V) {
 #pragma unroll
                 for (int i = 0; i < epb; ++i)
@@ -239,7 +240,14 @@ __global__ __launch_bounds__(kLpThreads) __attribute__((amdgpu_waves_per_eu(C <=
                 int tq = tid;  // (recomputed, not kept live across the loop)
                 asm volatile("" : "+v"(tq));
                 const uint4 kk = reinterpret_cast<const uint4*>(s_tkey)[tq];
-                const uint32_t k4[4] = {kk.x, kk.y, kk.z, kk.w};
+                uint32_t k4[4] = {kk.x, kk.y, kk.z, kk.w};
+                if constexpr (NT == 2 * kLpThreads) {  // 256 maxima, each of two threads
+                    const uint4 k2 = reinterpret_cast<const uint4*>(s_tkey + kLpThreads)[tq];
+                    k4[0] = max(k4[0], k2.x);
+                    k4[1] = max(k4[1], k2.y);
+                    k4[2] = max(k4[2], k2.z);
+                    k4[3] = max(k4[3], k2.w);
+                }
                 float th;
                 if constexpr (DT == 0) {
                     th = key_value(mth_largest_key<32>(k4, M));
@@ -274,7 +282,7 @@ __global__ __launch_bounds__(kLpThreads) __attribute__((amdgpu_waves_per_eu(C <=
                     const int slot = atomicAdd(&s_nblk, 1);
                     if (slot < kLpBlockCap) {
                         s_blk[slot] = d[c];
-                        s_blk_v0[slot] = vt + c * kLpThreads * epb;
+                        s_blk_v0[slot] = vt + c * NT * epb;
                     }
                 }
             }
@@ -296,12 +304,12 @@ __global__ __launch_bounds__(kLpThreads) __attribute__((amdgpu_waves_per_eu(C <=
         const bool mask_eos_n = s_slot_mask_eos != 0;
         const int eos_n = s_slot_eos;
         constexpr int kLate = C >= 16 ? 4 : 0;
-        const int lead_n = load_row<DT, C, 0, C - kLate>(p, rn, rn < rows, tid, d);
+        const int lead_n = load_row<NT, DT, C, 0, C - kLate>(p, rn, rn < rows, tid, d);
 #pragma unroll
         for (int e = 0; e < epb; ++e) asm volatile("" : "+v"(ban_by[e])::"memory");
 
         if (keep) {
-            for (int i = tid; i < nblk_hit; i += kLpThreads) {
+            for (int i = tid; i < nblk_hit; i += NT) {
                 const v4u32 blk = s_blk[i];
                 const int v0 = s_blk_v0[i];
                 uint32_t ban = 0;
@@ -336,7 +344,7 @@ __global__ __launch_bounds__(kLpThreads) __attribute__((amdgpu_waves_per_eu(C <=
         const bool listed = keep && n <= kSurvivorCap;
         if (listed) {
             ShortEntry* out = p.shortlist + r * M;
-            for (int i = tid; i < n; i += kLpThreads) {
+            for (int i = tid; i < n; i += NT) {
                 const uint64_t ki = s_key[i];
                 int rank = 0;
                 int j = 0;
@@ -372,7 +380,7 @@ __global__ __launch_bounds__(kLpThreads) __attribute__((amdgpu_waves_per_eu(C <=
             if (tid == 0) publish_rowinfo(p.rowinfo + r, info, coherent);
             signal_row_done(p, r, tid);
         }
-        if constexpr (kLate > 0) load_row<DT, C, C - kLate, C>(p, rn, rn < rows, tid, d);
+        if constexpr (kLate > 0) load_row<NT, DT, C, C - kLate, C>(p, rn, rn < rows, tid, d);
         r = rn;
         b = bn;
         mask_eos = mask_eos_n;
@@ -386,7 +394,8 @@ __global__ __launch_bounds__(kLpThreads) __attribute__((amdgpu_waves_per_eu(C <=
 int logprob_blocks(const DecodeParams& p) {
     const int64_t esz = p.dtype == 0 ? 4 : 2;
     const int64_t nblk = (15 + static_cast<int64_t>(p.V) * esz + 15) / 16;
-    return static_cast<int>((nblk + kLpThreads - 1) / kLpThreads);
+    const int64_t per = (nblk + kLpThreads - 1) / kLpThreads;
+    return per > 4 * kLpMaxBlocks ? 4 * kLpMaxBlocks : static_cast<int>(per);
 }
 
 }  // namespace
@@ -394,7 +403,7 @@ int logprob_blocks(const DecodeParams& p) {
 bool row_logprob_eligible(const DecodeParams& p) {
     if (p.from_logits) return false;
     if (p.M > 256) return false;
-    return logprob_blocks(p) <= kLpMaxBlocks;
+    return logprob_blocks(p) <= 2 * kLpMaxBlocks;
 }
 
 namespace {
@@ -402,24 +411,23 @@ namespace {
 int g_lp_cus[64];
 
 // Resident workgroups of one instantiation per CU (every gfx950 the same).
-template <int DT, int C>
+template <int DT, int C, int NT>
 int lp_per_cu() {
     static const int n = [] {
         int blocks = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(&row_logprob_kernel<DT, C>),
-                                                         kLpThreads, 0) != hipSuccess || blocks < 1)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(&row_logprob_kernel<DT, C, NT>),
+                                                         NT, 0) != hipSuccess || blocks < 1)
             blocks = 1;
         return blocks;
     }();
     return n;
 }
 
-template <int DT, int C>
+template <int DT, int C, int NT>
 hipError_t launch_lp(const DecodeParams& p, int64_t rows, int cus, hipStream_t stream) {
-    const int64_t slots = static_cast<int64_t>(cus) * lp_per_cu<DT, C>();
+    const int64_t slots = static_cast<int64_t>(cus) * lp_per_cu<DT, C, NT>();
     const int64_t grid = rows < slots ? rows : slots;
-    hipLaunchKernelGGL((row_logprob_kernel<DT, C>), dim3(static_cast<unsigned>(grid)), dim3(kLpThreads), 0, stream, p,
-                       rows);
+    hipLaunchKernelGGL((row_logprob_kernel<DT, C, NT>), dim3(static_cast<unsigned>(grid)), dim3(NT), 0, stream, p, rows);
     return hipGetLastError();
 }
 
@@ -442,22 +450,29 @@ hipError_t launch_row_logprob(const DecodeParams& p, int64_t rows, hipStream_t s
     }
     const int held = p.select_hold ? p.reserve_cus : 0;
     const int cus = g_lp_cus[device] - held > 0 ? g_lp_cus[device] - held : 1;
-#define DBS_LP_CASE(CB)                                                       \
-    if (need <= CB) {                                                         \
-        if (p.dtype == 0) return launch_lp<0, CB>(p, rows, cus, stream);      \
-        if (p.dtype == 1) return launch_lp<1, CB>(p, rows, cus, stream);      \
-        return launch_lp<2, CB>(p, rows, cus, stream);                        \
+#define DBS_LP_CASE(CB, NT)                                                       \
+    if (need <= CB * (NT / kLpThreads)) {                                         \
+        if (p.dtype == 0) return launch_lp<0, CB, NT>(p, rows, cus, stream);      \
+        if (p.dtype == 1) return launch_lp<1, CB, NT>(p, rows, cus, stream);      \
+        return launch_lp<2, CB, NT>(p, rows, cus, stream);                        \
     }
-    DBS_LP_CASE(2)
-    DBS_LP_CASE(4)
-    DBS_LP_CASE(8)
-    DBS_LP_CASE(12)
-    DBS_LP_CASE(16)
-    DBS_LP_CASE(20)
-    DBS_LP_CASE(24)
-    DBS_LP_CASE(28)
-    DBS_LP_CASE(32)
-    DBS_LP_CASE(40)
+    DBS_LP_CASE(2, kLpThreads)
+    DBS_LP_CASE(4, kLpThreads)
+    DBS_LP_CASE(8, kLpThreads)
+    DBS_LP_CASE(12, kLpThreads)
+    DBS_LP_CASE(16, kLpThreads)
+    DBS_LP_CASE(20, kLpThreads)
+    DBS_LP_CASE(24, kLpThreads)
+    DBS_LP_CASE(28, kLpThreads)
+    DBS_LP_CASE(32, kLpThreads)
+    DBS_LP_CASE(40, kLpThreads)
+    DBS_LP_CASE(46, kLpThreads)
+    DBS_LP_CASE(52, kLpThreads)
+    // rows past 53232 float32 (106480 16-bit) entries: 512 threads, one
+    // workgroup per CU
+    DBS_LP_CASE(32, 2 * kLpThreads)
+    DBS_LP_CASE(40, 2 * kLpThreads)
+    DBS_LP_CASE(52, 2 * kLpThreads)
 #undef DBS_LP_CASE
     return hipErrorInvalidValue;
 }

@@ -132,7 +132,7 @@ __device__ void row_pass_one(const DecodeParams& p, int64_t r, int b, int new_le
     }
     __syncthreads();
 
-    finish_row_wave<LOGITS, false>(p, r, lse, theta, any_bad, s_key, s_x, s_count, lane, b, mask_eos);
+    finish_row_wave<LOGITS>(p, r, lse, theta, any_bad, s_key, s_x, s_count, lane);
 }
 
 template <int DT, bool LOGITS, bool VEC>
@@ -153,30 +153,24 @@ std::atomic<int> g_row_pass_kind{-1};
 namespace {
 
 // The kernel of a row pass. Log-prob rows: the one-read kernel up to its
-// register limit. Logits: the relay kernel for the bfloat16 rows it fills, the
-// two-read stream kernel for every other row (row pass of 16 x 64 x 4 x 50257
-// f32: 487 us on the two-pass kernel, 280 on the stream kernel; 8 x 32 x 8 x
-// 128256 f16: 1790 resident, 214 stream; 32 x 48 x 5 x 50257 bf16: 618
-// pipelined, 326 stream; bf16 rows of 8000, 32000 and 100000: 1485, 727 and
-// 379 resident, 266, 243 and 289 stream). A forced kind that does not apply
-// falls back to the two-pass kernel.
-enum Kernel { kTwoPass, kResident, kPipe, kLogprob, kRelay, kStream };
+// register limit (16 x 64 x 4 x 50000 f32: 345 us on the two-pass kernel, 264
+// on the stream kernel, 152). Logits: the relay kernel for the bfloat16 rows it
+// fills. Every other row: the stream kernel (row pass of 16 x 64 x 4 x 50257
+// f32 logits 280 us, 487 on the two-pass kernel; 8 x 32 x 8 x 128256 f16 214,
+// 1115; f32 log-prob rows of 128256 307, 708). A forced kind that does not
+// apply, or is no longer a kernel of its own, takes the two-pass kernel.
+enum Kernel { kTwoPass, kLogprob, kRelay, kStream };
 Kernel row_kernel(const DecodeParams& p) {
     const int kind = g_row_pass_kind.load(std::memory_order_relaxed);
     if ((kind == -1 || kind == 3) && row_logprob_eligible(p)) return kLogprob;
     if ((kind == 5 || (kind == -1 && row_relay_preferred(p))) && row_relay_eligible(p)) return kRelay;
     if ((kind == -1 || kind == 7) && row_stream_eligible(p)) return kStream;
-    if ((kind == -1 || kind == 1) && row_resident_eligible(p)) return kResident;
-    if ((kind == -1 || kind == 2) && row_pipe_eligible(p)) return kPipe;
     return kTwoPass;
 }
 
 }  // namespace
 
-bool row_pass_persistent(const DecodeParams& p) {
-    const Kernel k = row_kernel(p);
-    return k == kRelay || k == kResident || k == kPipe;
-}
+bool row_pass_persistent(const DecodeParams& p) { return row_kernel(p) == kRelay; }
 
 hipError_t launch_row_pass(const DecodeParams& p, hipStream_t stream) {
     const int64_t rows = p.step_mode ? static_cast<int64_t>(p.B) * p.K : static_cast<int64_t>(p.B) * p.T * p.K;
@@ -188,8 +182,6 @@ hipError_t launch_row_pass(const DecodeParams& p, hipStream_t stream) {
         case kLogprob: return launch_row_logprob(p, rows, stream);
         case kRelay: return launch_row_relay(p, rows, stream);
         case kStream: return launch_row_stream(p, rows, stream);
-        case kResident: return launch_row_resident(p, rows, stream);
-        case kPipe: return launch_row_pipe(p, rows, stream);
         case kTwoPass: break;
     }
     const dim3 grid(static_cast<unsigned>(rows));

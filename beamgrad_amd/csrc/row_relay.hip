@@ -729,7 +729,10 @@ bool row_relay_eligible(const DecodeParams& p) {
     return p.M <= 256;
 }
 
-bool row_relay_preferred(const DecodeParams& p) { return (p.V + 255) / 256 >= (3 * kRlStripes) / 4; }
+// From 352 stripes on: below, the stream pass costs less (16 x 32 x 8 rows of
+// 88064: 250 us here, 246 there; of 95232: 247 and 259), as a row here costs
+// what its 32 chunks hold whatever its length.
+bool row_relay_preferred(const DecodeParams& p) { return (p.V + 255) / 256 >= 352; }
 
 hipError_t launch_row_relay(const DecodeParams& p, int64_t rows, hipStream_t stream) {
     int device = 0;

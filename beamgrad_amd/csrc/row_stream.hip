@@ -1,8 +1,9 @@
 // SPDX-License-Identifier: MIT
 //
-// Row pass for logits that reads a row twice: 32-bit and binary16 rows of any
-// size and alignment, and the bfloat16 rows the register-resident passes do
-// not take.
+// Row pass that reads a row twice, for rows of any type, size and alignment:
+// the logits rows the relay pass does not take, and log-prob rows past the
+// one-read pass's registers (which have no logsumexp: the second read only
+// finds the survivors).
 //
 // Each row's logsumexp folds exp(fl(x - max)) into 256 lanes (lane j = v mod
 // 256, increasing v; reference src/kernels_scalar.cpp:48-66), so the maximum
@@ -25,8 +26,8 @@
 // 7.2 TB/s read once), and binary16 and float32 terms cost 25 vector operations
 // each (exp_term), 28 an element with the first read's: 2.9 TB/s of binary16
 // and 5.8 TB/s of float32 rows at 2.4 GHz. Keeping the row on chip instead
-// pays only where the arithmetic leaves room: bfloat16 rows (a table of the
-// terms), which the relay and resident passes take where alignment allows.
+// pays only where the arithmetic leaves room: long bfloat16 rows (a table of the
+// terms), which the relay pass takes where alignment allows.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -144,10 +145,10 @@ struct Extremes {
     }
 };
 
-template <int DT>
-__global__ __launch_bounds__(kStThreads) __attribute__((amdgpu_waves_per_eu(4))) void row_stream_kernel(DecodeParams p,
-                                                                                                       int64_t rows) {
-    __shared__ __align__(16) float s_lut[DT == 2 ? 2 * kLutHalf : 1];
+template <int DT, bool LOGITS>
+__global__ __launch_bounds__(kStThreads) __attribute__((amdgpu_waves_per_eu(DT == 2 && LOGITS ? 3 : 4))) void
+row_stream_kernel(DecodeParams p, int64_t rows) {
+    __shared__ __align__(16) float s_lut[DT == 2 && LOGITS ? 2 * kLutHalf : 1];
     __shared__ uint64_t s_key[kSurvivorCap];
     __shared__ float s_x[kSurvivorCap];
     __shared__ uint32_t s_rec[kStRecords];
@@ -261,13 +262,13 @@ __global__ __launch_bounds__(kStThreads) __attribute__((amdgpu_waves_per_eu(4)))
         __syncthreads();
         if (tid == kTicketThread) s_bad = 0;  // every thread has read it
         const float m = s_m;
-        const bool do_lse = m > -kInf;
+        const bool do_lse = m > -kInf;  // (log-probs: a finite entry)
         // no shortlist: a flagged row, or one whose every element would survive
         const bool listing = M > 0 && !any_bad && s_theta > -kInf;
         const float theta = listing ? s_theta : kInf;
 
         bool table = false;
-        if constexpr (DT == 2) {
+        if constexpr (DT == 2 && LOGITS) {
             // terms by bfloat16 pattern (term_slots), where the row fits the
             // table and is long enough to pay for its 8192 terms
             table = V >= kStTableRow && table_fits_fixed(m);
@@ -303,8 +304,10 @@ __global__ __launch_bounds__(kStThreads) __attribute__((amdgpu_waves_per_eu(4)))
 #pragma unroll
             for (int u = 3; u + 1 < kStGroup; u += 2) gm = max3(gm, x[u], x[u + 1]);
             gm = max3(gm, x[kStGroup - 1], x[kStGroup - 1]);
+            if constexpr (LOGITS) {
 #pragma unroll
-            for (int u = 0; u < kStGroup; ++u) acc = acc + exp_term(m, x[u]);
+                for (int u = 0; u < kStGroup; ++u) acc = acc + exp_term(m, x[u]);
+            }
             record(gm, g);
         };
         auto fold_table = [&](const uint32_t (&h)[kStGroup], int g, auto edge) __attribute__((always_inline)) {
@@ -366,8 +369,8 @@ __global__ __launch_bounds__(kStThreads) __attribute__((amdgpu_waves_per_eu(4)))
                 one(h0, g, std::true_type{});
             }
         };
-        if (do_lse) {
-            if (DT == 2 && table) fold_row(fold_table);
+        if (do_lse && (LOGITS || listing)) {
+            if (DT == 2 && LOGITS && table) fold_row(fold_table);
             else fold_row(fold);
         }
         s_acc[tid] = acc;
@@ -378,10 +381,13 @@ __global__ __launch_bounds__(kStThreads) __attribute__((amdgpu_waves_per_eu(4)))
         const int nrec = s_nrec;
         const bool keep = listing && nrec <= kStRecords;
         if (tid < 64) {
-            float a[4];
+            float lse = 0.0f;
+            if constexpr (LOGITS) {
+                float a[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) a[e] = s_acc[4 * tid + e];
-            const float lse = do_lse ? logsumexp_from(m, lane_tree_sum(a, tid)) : -kInf;
+                for (int e = 0; e < 4; ++e) a[e] = s_acc[4 * tid + e];
+                lse = do_lse ? logsumexp_from(m, lane_tree_sum(a, tid)) : -kInf;
+            }
             if (tid == 0) s_lse = lse;
         } else if (keep) {
             const bool mask_eos = new_len < min_length_of(p, b);
@@ -423,7 +429,7 @@ __global__ __launch_bounds__(kStThreads) __attribute__((amdgpu_waves_per_eu(4)))
                 for (; j < n; ++j) rank += static_cast<int>(s_key[j] > ki);
                 if (rank < M) {
                     const int32_t tok = static_cast<int32_t>(0xffffffffu - static_cast<uint32_t>(ki & 0xffffffffu));
-                    publish_entry(out, rank, s_x[i] - lse, tok, coherent);
+                    publish_entry(out, rank, LOGITS ? s_x[i] - lse : s_x[i], tok, coherent);
                 } else if (rank == M) {
                     s_bound = s_x[i];
                 }
@@ -436,10 +442,11 @@ __global__ __launch_bounds__(kStThreads) __attribute__((amdgpu_waves_per_eu(4)))
             info.invalid = any_bad ? 1u : 0u;
             info.bound = -kInf;
             info.count = 0;
-            if (M > 0 && do_lse) {
+            if (M > 0 && (do_lse || !LOGITS)) {
                 if (listed) {
                     info.count = n < M ? n : M;
-                    info.bound = (n > M ? s_bound : theta) - lse;
+                    info.bound = n > M ? s_bound : theta;
+                    if constexpr (LOGITS) info.bound = info.bound - lse;
                 } else {
                     info.count = -1;
                 }
@@ -455,18 +462,19 @@ __global__ __launch_bounds__(kStThreads) __attribute__((amdgpu_waves_per_eu(4)))
 
 int g_st_cus[64];
 
-template <int DT>
+template <int DT, bool LOGITS>
 hipError_t launch_st(const DecodeParams& p, int64_t rows, int cus, hipStream_t stream) {
     static const int per_cu = [] {
         int blocks = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(&row_stream_kernel<DT>),
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(&row_stream_kernel<DT, LOGITS>),
                                                          kStThreads, 0) != hipSuccess || blocks < 1)
             blocks = 1;
         return blocks;
     }();
     const int64_t slots = static_cast<int64_t>(cus) * per_cu;
     const int64_t grid = rows < slots ? rows : slots;
-    hipLaunchKernelGGL((row_stream_kernel<DT>), dim3(static_cast<unsigned>(grid)), dim3(kStThreads), 0, stream, p, rows);
+    hipLaunchKernelGGL((row_stream_kernel<DT, LOGITS>), dim3(static_cast<unsigned>(grid)), dim3(kStThreads), 0, stream, p,
+                       rows);
     return hipGetLastError();
 }
 
@@ -474,7 +482,7 @@ hipError_t launch_st(const DecodeParams& p, int64_t rows, int cus, hipStream_t s
 
 bool row_stream_eligible(const DecodeParams& p) {
     // (byte offsets within a row are 31-bit, with room for the last group)
-    return p.from_logits && p.M <= 256 && p.V < (1 << 28);
+    return p.M <= 256 && p.V < (1 << 28);
 }
 
 hipError_t launch_row_stream(const DecodeParams& p, int64_t rows, hipStream_t stream) {
@@ -491,11 +499,14 @@ hipError_t launch_row_stream(const DecodeParams& p, int64_t rows, hipStream_t st
     }
     const int held = p.select_hold ? p.reserve_cus : 0;
     const int cus = g_st_cus[device] - held > 0 ? g_st_cus[device] - held : 1;
+#define DBS_ST_CASE(DT) \
+    return p.from_logits ? launch_st<DT, true>(p, rows, cus, stream) : launch_st<DT, false>(p, rows, cus, stream)
     switch (p.dtype) {
-        case 0: return launch_st<0>(p, rows, cus, stream);
-        case 1: return launch_st<1>(p, rows, cus, stream);
-        default: return launch_st<2>(p, rows, cus, stream);
+        case 0: DBS_ST_CASE(0);
+        case 1: DBS_ST_CASE(1);
+        default: DBS_ST_CASE(2);
     }
+#undef DBS_ST_CASE
 }
 
 }  // namespace dbs_hip

@@ -232,13 +232,12 @@ DBS_CUDA_EXPORT int dbs_hip_profile_read(int kernel, double* total_ms, int64_t* 
 
 /* Row-pass kernel choice for tests and measurements (no counterpart in the
  * reference; every choice gives the same results): -1 automatic (the
- * default: for log-prob rows the one-read log-prob kernel where it applies,
- * else the resident or the pipelined 16-bit kernel, else the two-pass kernel;
- * for logits the relay kernel for the bfloat16 rows it fills, else the
- * stream kernel), 0 two-pass, 1 resident 16-bit (V % 8 == 0, 16-byte aligned
- * rows), 2 pipelined 16-bit (any V), 3 one-read log-prob rows (any dtype, rows
- * up to 163824 bytes), 5 relay for bfloat16 logits (V % 8 == 0, 16-byte aligned
- * rows, V <= 155648), 7 stream (logits, any dtype and V); 4 and 6 are not
+ * default: for log-prob rows the one-read log-prob kernel where it applies;
+ * for logits the relay kernel for the bfloat16 rows it fills; for every other
+ * row the stream kernel), 0 two-pass, 3 one-read log-prob rows (any dtype, rows
+ * up to 425968 bytes), 5 relay for bfloat16 logits (V % 8 == 0, 16-byte aligned
+ * rows, V <= 155648), 7 stream (any dtype and V); 1 and 2 are accepted and
+ * take the two-pass kernel; 4 and 6 are not
  * kernels (-2). A kernel that does not apply to a decode falls back to the
  * two-pass one. Returns the previous choice, or -2 for an invalid
  * argument. */

@@ -100,3 +100,27 @@ def test_stream_long_shortlists(hip, oracle, stream, dtype):
     x = rng.normal(0.0, 1.0, size=(2, 3, 64, 5003)).astype(np.float32)
     banned = (rng.random(5003) < 0.3).astype(np.uint8)
     _check(hip, oracle, to_bits(x, dtype), dtype, from_logits=True, alpha=0.6, banned=banned)
+
+
+@pytest.mark.parametrize("dtype,V", [("f32", 1), ("f32", 4097), ("f32", 20483), ("f16", 8191), ("bf16", 12289)])
+def test_stream_log_probs(hip, oracle, stream, dtype, V):
+    rng = np.random.default_rng(V)
+    x = rng.normal(-9.0, 2.0, size=(2, 4, 3, V)).astype(np.float32)
+    x[rng.random(x.shape) < 0.05] = -np.inf
+    x[1, 2, 0, V // 2] = np.nan  # read: the row is flagged and read in full
+    for offset in (0, 1):
+        _check(hip, oracle, to_bits(x, dtype), dtype, eos_token=-1, alpha=0.6, x_offset=offset)
+
+
+# around the log-prob row pass's blocks per thread: 40, 46 and 52 of 256
+# threads, 32, 40 and 52 of 512, and past them (the stream pass)
+@pytest.mark.parametrize("dtype,V", [("f32", 40957), ("f32", 47100), ("f32", 53233), ("f32", 65533), ("f32", 81918),
+                                     ("f32", 106480), ("f32", 106489), ("f16", 81913), ("bf16", 106481),
+                                     ("f16", 131069), ("bf16", 151936), ("f16", 212960), ("bf16", 212977)])
+def test_long_log_prob_rows(hip, oracle, dtype, V):
+    rng = np.random.default_rng(V)
+    x = rng.normal(-12.0, 2.0, size=(2, 3, 3, V)).astype(np.float32)
+    x[1, 1, 1, 5] = np.inf  # flagged where read
+    x[0, :, :, V - 1] = -3.0  # the last element is selected
+    for offset in (0, 3):
+        _check(hip, oracle, to_bits(x, dtype), dtype, eos_token=-1, alpha=0.6, x_offset=offset)
