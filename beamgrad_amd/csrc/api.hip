@@ -17,6 +17,7 @@
 #include "dbs_cuda.h"
 #include "dbs_hip.h"
 #include "engine.hpp"
+#include "torch_engine.hpp"
 #include "host_entry.hpp"
 
 using namespace dbs_hip;
@@ -855,6 +856,38 @@ DBS_CUDA_EXPORT int dbs_hip_backtrack(const int32_t* tokens, const int32_t* pare
     hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
     return finish(stream,
                   launch_backtrack(tokens, parents, steps_per_example, batch_size, steps, beam_size, sequences, stream));
+}
+
+int beamgrad_advance_beams(const int32_t* tokens, const int32_t* parents, const int32_t* lengths,
+                           const float* raw_scores, const uint8_t* from_logprob, const uint8_t* finished,
+                           const int64_t* sequences, int batch_size, int beam_size, int step, int64_t* sequences_out,
+                           int32_t* prefixes_out, int64_t* tokens64, int64_t* parents64, int64_t* lengths64,
+                           uint8_t* finished_bool, uint8_t* active, int32_t* any_active, void* stream_ptr) {
+    if (!tokens || !parents || !lengths || !raw_scores || !from_logprob || !finished || (step > 0 && !sequences) ||
+        !sequences_out || !prefixes_out || !tokens64 || !parents64 || !lengths64 || !finished_bool || !active ||
+        !any_active || batch_size <= 0 || beam_size <= 0 || step < 0 || step == INT32_MAX)
+        return DBS_CUDA_STATUS_INVALID_ARGUMENT;
+    AdvanceBeams a{};
+    a.tokens = tokens;
+    a.parents = parents;
+    a.lengths = lengths;
+    a.raw = raw_scores;
+    a.flp = from_logprob;
+    a.finished = finished;
+    a.sequences = sequences;
+    a.sequences_out = sequences_out;
+    a.prefixes_out = prefixes_out;
+    a.tokens64 = tokens64;
+    a.parents64 = parents64;
+    a.lengths64 = lengths64;
+    a.finished_bool = finished_bool;
+    a.active = active;
+    a.any_active = any_active;
+    a.beams = static_cast<int64_t>(batch_size) * beam_size;
+    a.K = beam_size;
+    a.t = step;
+    hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
+    return finish(stream, launch_advance_beams(a, stream));
 }
 
 DBS_CUDA_EXPORT int dbs_hip_widen_trace(const int32_t* final_lengths, const int32_t* tokens, const int32_t* parents,

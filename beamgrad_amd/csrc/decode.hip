@@ -76,6 +76,39 @@ __global__ __launch_bounds__(256) void widen_trace_kernel(WidenTrace w) {
     for (int64_t i = first; i < w.n_steps; i += stride) w.steps64[i] = w.steps ? w.steps[i] : w.T;
 }
 
+// One thread per token of the new sequences; block 0 also takes the beams'
+// own values. A launch in place of some twenty elementwise ones per step.
+__global__ __launch_bounds__(256) void advance_beams_kernel(AdvanceBeams a) {
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * 256;
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    const int L = a.t + 1;
+    for (int64_t i = first; i < a.beams * L; i += stride) {
+        const int64_t beam = i / L;
+        const int at = static_cast<int>(i - beam * L);
+        const int parent = a.parents[beam];
+        int64_t v = -1;
+        if (parent >= 0 && at < a.t) v = a.sequences[(beam - beam % a.K + parent) * a.t + at];
+        else if (parent >= 0 && a.flp[beam] != 0) v = a.tokens[beam];
+        a.sequences_out[i] = v;
+        a.prefixes_out[i] = static_cast<int32_t>(v);
+    }
+    if (blockIdx.x != 0) return;
+    __shared__ int any;
+    if (threadIdx.x == 0) any = 0;
+    __syncthreads();
+    for (int64_t i = threadIdx.x; i < a.beams; i += 256) {
+        const float raw = a.raw[i];
+        const bool active = raw < kInf && raw > -kInf && a.finished[i] == 0;
+        a.tokens64[i] = a.tokens[i];
+        a.parents64[i] = a.parents[i];
+        a.lengths64[i] = a.lengths[i];
+        a.finished_bool[i] = a.finished[i] != 0 ? 1 : 0;
+        a.active[i] = active ? 1 : 0;
+        if (active) any = 1;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) *a.any_active = any;
+}
 
 __global__ void length_penalty_kernel(const int32_t* lengths, int64_t n, float alpha, float* out) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -459,6 +492,13 @@ hipError_t launch_widen_trace(const WidenTrace& w, hipStream_t stream) {
     return hipGetLastError();
 }
 
+
+hipError_t launch_advance_beams(const AdvanceBeams& a, hipStream_t stream) {
+    const int64_t blocks = (a.beams * (a.t + 1) + 255) / 256;
+    hipLaunchKernelGGL(advance_beams_kernel, dim3(static_cast<unsigned>(blocks < 2048 ? blocks : 2048)), dim3(256), 0,
+                       stream, a);
+    return hipGetLastError();
+}
 
 hipError_t launch_length_penalty(const int32_t* lengths, int64_t n, float alpha, float* out, hipStream_t stream) {
     if (n <= 0) return hipSuccess;

@@ -245,6 +245,26 @@ struct WidenTrace {
     int T;
 };
 hipError_t launch_widen_trace(const WidenTrace& w, hipStream_t stream);
+
+// The beams after one step, as a stepping loop keeps them: the step's int32 /
+// uint8 outputs [B, K] widened for torch, each beam's tokens [B, K, t + 1]
+// (its parent's, then the one it emitted, -1 where it emitted none; a dead slot
+// all -1) in both index types, which beams the next step reads, and whether
+// there are any.
+struct AdvanceBeams {
+    const int32_t *tokens, *parents, *lengths;
+    const float* raw;
+    const uint8_t *flp, *finished;
+    const int64_t* sequences;  // [B, K, t]
+    int64_t *sequences_out;    // [B, K, t + 1]
+    int32_t* prefixes_out;     // [B, K, t + 1]
+    int64_t *tokens64, *parents64, *lengths64;
+    uint8_t *finished_bool, *active;
+    int32_t* any_active;
+    int64_t beams;             // B * K
+    int K, t;
+};
+hipError_t launch_advance_beams(const AdvanceBeams& a, hipStream_t stream);
 // The read-back that ends a decode: `bytes` bytes at `src` (written only by
 // the decode's select pass: its flags or its fault word) copied to `dst` on
 // the host through pinned memory, waiting for nothing else. After an
