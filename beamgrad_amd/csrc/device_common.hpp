@@ -243,13 +243,14 @@ __device__ __forceinline__ void signal_row_done(const DecodeParams& p, int64_t r
 // most significant bit: each round counts, with ballots, the keys that agree
 // with the bits decided so far and have the next bit set, and keeps that half
 // when it holds at least the rank still sought. Exact, ties included, and the
-// same in every lane; no LDS and no lane exchange besides the ballots.
-template <int BITS>
+// same in every lane; no LDS and no lane exchange besides the ballots. LOW:
+// the key's low LOW bits are left zero (at least M keys reach it).
+template <int BITS, int LOW = 0>
 __device__ __forceinline__ uint32_t mth_largest_key(const uint32_t (&k)[4], int M) {
     uint32_t prefix = 0;
     int need = M;
 #pragma unroll
-    for (int bit = BITS - 1; bit >= 0; --bit) {
+    for (int bit = BITS - 1; bit >= LOW; --bit) {
         const uint32_t want = (prefix >> bit) | 1u;
         int c = 0;
 #pragma unroll

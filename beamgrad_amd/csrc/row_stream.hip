@@ -40,7 +40,9 @@ namespace {
 
 constexpr int kStThreads = 256;
 constexpr int kStGroup = 16;    // stripes per group
-constexpr int kStRecords = 512; // groups holding survivors, at most (else the row is read in full)
+// LDS beside the 32 KB term table: four workgroups per CU take 40 KB each.
+constexpr int kStRecords = 432;   // groups holding survivors, at most (else the row is read in full)
+constexpr int kStSurvivors = 432; // survivors, at most (likewise)
 constexpr int kStTableRow = 12000;  // bfloat16 rows from which the term table pays (8192 terms against 5 of 25 operations an element)
 constexpr int kStBlocks = 8;    // 16-byte loads in flight per thread in the first read
 constexpr int kFirstPolicy = 0, kSecondPolicy = 2;  // (the second read streams: 4.0 against 3.7 TB/s)
@@ -145,15 +147,16 @@ struct Extremes {
     }
 };
 
-template <int DT, bool LOGITS>
-__global__ __launch_bounds__(kStThreads) __attribute__((amdgpu_waves_per_eu(DT == 2 && LOGITS ? 3 : 4))) void
+// TABLE: bfloat16 logits rows long enough for the term table.
+template <int DT, bool LOGITS, bool TABLE>
+__global__ __launch_bounds__(kStThreads) __attribute__((amdgpu_waves_per_eu(4))) void
 row_stream_kernel(DecodeParams p, int64_t rows) {
-    __shared__ __align__(16) float s_lut[DT == 2 && LOGITS ? 2 * kLutHalf : 1];
-    __shared__ uint64_t s_key[kSurvivorCap];
-    __shared__ float s_x[kSurvivorCap];
+    __shared__ __align__(16) float s_lut[TABLE ? 2 * kLutHalf : 1];
+    __shared__ uint64_t s_key[kStSurvivors];
+    __shared__ float s_x[kStSurvivors];
     __shared__ uint32_t s_rec[kStRecords];
-    __shared__ __align__(16) float s_acc[kStThreads];
     __shared__ __align__(16) uint32_t s_tkey[kStThreads];
+    float* const s_acc = reinterpret_cast<float*>(s_tkey);  // (the keys are read before the sums are written)
     __shared__ RowSlot s_slot;
     __shared__ int s_count, s_nrec, s_bad;
     __shared__ float s_m, s_theta, s_lse, s_bound;
@@ -234,6 +237,15 @@ row_stream_kernel(DecodeParams p, int64_t rows) {
             __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(a0 - lead2), 0, lead2 + V * esz, 0x00020000);
         const int voff = lead2 + tid * esz;
         const int S = (V + 255) >> 8;  // stripes
+        auto load_group = [&](uint32_t (&h)[kStGroup], int g) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < kStGroup; ++u)
+                h[u] = load_raw<DT>(rs, voff, min((g * kStGroup + u) * 256 * esz, lead2 + V * esz));
+        };
+        // (the scalar offset is kept within the view: past it, every lane's load
+        // is out of range and returns zero)
+        uint32_t h0[kStGroup];  // the first group goes out while the threshold and the table are made
+        load_group(h0, 0);
         if (any_bad) {
             // a row with NaN or +inf: the maximum of the entries below +inf
             tmax = -kInf;
@@ -249,7 +261,9 @@ row_stream_kernel(DecodeParams p, int64_t rows) {
             const uint32_t k4[4] = {kk.x, kk.y, kk.z, kk.w};
             const uint32_t top = max(max(kk.x, kk.y), max(kk.z, kk.w));
             const float m = wave_max_dpp(key_value(top));
-            const float th = M > 0 ? key_value(mth_largest_key<32>(k4, M)) : -kInf;
+            // (to its 20 highest bits, rounded down: at least M elements reach
+            // it, and twelve rounds less are waited for)
+            const float th = M > 0 ? key_value(mth_largest_key<32, 12>(k4, M)) : -kInf;
             if (tid == 0) {
                 s_m = m;
                 s_theta = th;
@@ -268,10 +282,9 @@ row_stream_kernel(DecodeParams p, int64_t rows) {
         const float theta = listing ? s_theta : kInf;
 
         bool table = false;
-        if constexpr (DT == 2 && LOGITS) {
-            // terms by bfloat16 pattern (term_slots), where the row fits the
-            // table and is long enough to pay for its 8192 terms
-            table = V >= kStTableRow && table_fits_fixed(m);
+        if constexpr (TABLE) {
+            // terms by bfloat16 pattern (term_slots), where the row fits them
+            table = table_fits_fixed(m);
             if (table) {
 #pragma unroll 4
                 for (int i = tid; i < 2 * kLutHalf; i += kStThreads) {
@@ -340,19 +353,11 @@ row_stream_kernel(DecodeParams p, int64_t rows) {
             for (int u = 0; u < kStGroup; ++u) acc = acc + e[u];
             record(gm, g);
         };
-        auto load_group = [&](uint32_t (&h)[kStGroup], int g) __attribute__((always_inline)) {
-#pragma unroll
-            for (int u = 0; u < kStGroup; ++u)
-                h[u] = load_raw<DT>(rs, voff, min((g * kStGroup + u) * 256 * esz, lead2 + V * esz));
-        };
-        // (the scalar offset is kept within the view: past it, every lane's load
-        // is out of range and returns zero)
         // Whole groups two at a time, each one's loads in flight while the
         // other folds, then the rest (loads past the row return zeros).
         auto fold_row = [&](auto one) __attribute__((always_inline)) {
             const int G = V / (256 * kStGroup);
-            uint32_t h0[kStGroup], h1[kStGroup];
-            load_group(h0, 0);
+            uint32_t h1[kStGroup];
             int g = 0;
 #pragma unroll 1
             for (; g + 2 <= G; g += 2) {
@@ -370,7 +375,7 @@ row_stream_kernel(DecodeParams p, int64_t rows) {
             }
         };
         if (do_lse && (LOGITS || listing)) {
-            if (DT == 2 && LOGITS && table) fold_row(fold_table);
+            if (TABLE && table) fold_row(fold_table);
             else fold_row(fold);
         }
         s_acc[tid] = acc;
@@ -398,7 +403,7 @@ row_stream_kernel(DecodeParams p, int64_t rows) {
                 const float x = raw_value<DT>(load_raw<DT>(rs, lead2 + j * esz + s * 256 * esz, 0));
                 if (v < V && x >= theta && !static_masked(p, b, v, mask_eos)) {
                     const int slot = atomicAdd(&s_count, 1);
-                    if (slot < kSurvivorCap) {
+                    if (slot < kStSurvivors) {
                         s_key[slot] = survivor_key(x, v);
                         s_x[slot] = x;
                     }
@@ -414,7 +419,7 @@ row_stream_kernel(DecodeParams p, int64_t rows) {
         // before it (keys are distinct); ranks below M are written in place,
         // rank M is the bound on the rest.
         const int n = s_count;
-        const bool listed = keep && n <= kSurvivorCap;
+        const bool listed = keep && n <= kStSurvivors;
         if (listed) {
             ShortEntry* out = p.shortlist + r * M;
             for (int i = tid; i < n; i += kStThreads) {
@@ -462,18 +467,18 @@ row_stream_kernel(DecodeParams p, int64_t rows) {
 
 int g_st_cus[64];
 
-template <int DT, bool LOGITS>
+template <int DT, bool LOGITS, bool TABLE = false>
 hipError_t launch_st(const DecodeParams& p, int64_t rows, int cus, hipStream_t stream) {
     static const int per_cu = [] {
         int blocks = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(&row_stream_kernel<DT, LOGITS>),
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(&row_stream_kernel<DT, LOGITS, TABLE>),
                                                          kStThreads, 0) != hipSuccess || blocks < 1)
             blocks = 1;
         return blocks;
     }();
     const int64_t slots = static_cast<int64_t>(cus) * per_cu;
     const int64_t grid = rows < slots ? rows : slots;
-    hipLaunchKernelGGL((row_stream_kernel<DT, LOGITS>), dim3(static_cast<unsigned>(grid)), dim3(kStThreads), 0, stream, p,
+    hipLaunchKernelGGL((row_stream_kernel<DT, LOGITS, TABLE>), dim3(static_cast<unsigned>(grid)), dim3(kStThreads), 0, stream, p,
                        rows);
     return hipGetLastError();
 }
@@ -499,6 +504,7 @@ hipError_t launch_row_stream(const DecodeParams& p, int64_t rows, hipStream_t st
     }
     const int held = p.select_hold ? p.reserve_cus : 0;
     const int cus = g_st_cus[device] - held > 0 ? g_st_cus[device] - held : 1;
+    if (p.dtype == 2 && p.from_logits && p.V >= kStTableRow) return launch_st<2, true, true>(p, rows, cus, stream);
 #define DBS_ST_CASE(DT) \
     return p.from_logits ? launch_st<DT, true>(p, rows, cus, stream) : launch_st<DT, false>(p, rows, cus, stream)
     switch (p.dtype) {
