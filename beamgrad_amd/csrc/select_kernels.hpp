@@ -1611,10 +1611,125 @@ __device__ __forceinline__ void issue_tagged(const DecodeParams& p, int b, int t
     }
 }
 
-// The steps of an unconstrained decode of at most kGridBeams beams, the
-// candidates in a grid: lane (k, j) = k K + j holds entry j of beam k's
-// shortlist (only the first K of a list can be selected), and every lane of
-// beam k its state, so that a step moves nothing between lanes but the
+// The prefixes of a constrained decode's one-wavefront pass, in LDS: per beam
+// one record, a signature of its (n - 1)-grams but the last, one of its
+// tokens, and the tokens, in two buffers (the step's and the next). A new
+// beam's record is its parent's, copied 16 bytes a lane, a record a time (the
+// parent is wave-uniform: no per-lane address arithmetic, 5 x 128 tokens in 20
+// LDS operations), with the new token's bits set in place after.
+struct Prefixes {
+    uint32_t* rec;                // [2][K][R]
+    int32_t *blk, *nblk, *plen;   // [K][P] n-gram-blocked tokens, their counts, the lengths of beams that list them
+    int K, P, W, R, shift, cur;
+
+    __device__ __forceinline__ uint32_t* gram_sig(int k) const { return rec + (cur * K + k) * R; }
+    __device__ __forceinline__ uint32_t* token_sig(int k) const { return gram_sig(k) + W; }
+    __device__ __forceinline__ int32_t* tokens(int k) const { return reinterpret_cast<int32_t*>(gram_sig(k) + 2 * W); }
+    // Whether the two bits of v are set (if not, v was never added).
+    __device__ __forceinline__ bool maybe(const uint32_t* sig, int v) const {
+        const uint32_t h0 = sig_bit0(v, shift), h1 = sig_bit1(v, shift);
+        return (((sig[h0 >> 5] >> (h0 & 31u)) & (sig[h1 >> 5] >> (h1 & 31u))) & 1u) != 0u;
+    }
+    __device__ __forceinline__ void add(uint32_t* sig, int v) const {
+        const uint32_t h0 = sig_bit0(v, shift), h1 = sig_bit1(v, shift);
+        atomicOr(&sig[h0 >> 5], 1u << (h0 & 31u));
+        atomicOr(&sig[h1 >> 5], 1u << (h1 & 31u));
+    }
+    // The last n - 1 of beam k's len tokens, hashed (FNV-1a): the first four
+    // reads in flight together.
+    __device__ __forceinline__ uint32_t tail_hash(int k, int len, int n) const {
+        const int32_t* pre = tokens(k);
+        const int q0 = len - (n - 1);
+        uint32_t h = 0x811C9DC5u;
+        int32_t a[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) a[u] = pre[u < n - 1 ? q0 + u : 0];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (u < n - 1) h = (h ^ static_cast<uint32_t>(a[u])) * 0x01000193u;
+        for (int u = 4; u < n - 1; ++u) h = (h ^ static_cast<uint32_t>(pre[q0 + u])) * 0x01000193u;
+        return h;
+    }
+    // Each listing beam's blocked tokens (plen[k] its length, -1: none): those
+    // that followed an earlier occurrence of its last n - 1 tokens; nblk is
+    // zero. One lane per (beam k, position i), eight items per lane a round,
+    // every read of a round in flight together (beam k's positions at a
+    // power-of-two stride >= t: no division).
+    __device__ __forceinline__ void list_blocked(int n, int t, int lane) const {
+        const int Pt = min(P, t);
+        const int ps = Pt > 1 ? 32 - __builtin_clz(static_cast<uint32_t>(Pt - 1)) : 0, total = K << ps;
+        for (int j0 = 0; j0 < total; j0 += 8 * 64) {
+            int kk[8], ii[8], tl[8];
+            bool on[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int j = j0 + 64 * u + lane;
+                const int jc = j < total ? j : 0;
+                kk[u] = jc >> ps;
+                ii[u] = jc & ((1 << ps) - 1);
+                const int Lk = plen[kk[u]];
+                on[u] = j < total && ii[u] + n <= Lk;  // (a beam that lists none: -1)
+                tl[u] = on[u] ? Lk - (n - 1) : 0;
+            }
+            bool same[8] = {true, true, true, true, true, true, true, true};
+            for (int q = 0; q < n - 1; ++q) {
+                int32_t a[8], c[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int32_t* pre = tokens(kk[u]);
+                    a[u] = pre[on[u] ? ii[u] + q : 0];
+                    c[u] = pre[on[u] ? tl[u] + q : 0];
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) same[u] = same[u] && a[u] == c[u];
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                if (on[u] && same[u]) {
+                    const int slot = atomicAdd(&nblk[kk[u]], 1);
+                    blk[kk[u] * P + slot] = tokens(kk[u])[ii[u] + n - 1];
+                }
+            }
+        }
+    }
+    // The next buffer: beam k takes the record of its parent (par in lane k
+    // stride; none: any record, as it is never read), whose prefix holds at
+    // most t tokens; then, where `grows` (one lane of a beam k), token v at
+    // position at, and where `gram` the (n - 1)-gram hash gh.
+    __device__ __forceinline__ void advance(int par, int t, int lane, int stride, int k, bool grows, int v, int at,
+                                            bool gram, uint32_t gh, bool grams) {
+        const int first = grams ? 0 : W / 4, last = W / 2 + ((min(P, t) + 3) >> 2);
+        const uint4* src = reinterpret_cast<const uint4*>(rec + cur * K * R);
+        uint4* dst = reinterpret_cast<uint4*>(rec + (cur ^ 1) * K * R);
+        for (int c0 = first; c0 < last; c0 += 64) {
+            const int c = min(c0 + lane, last - 1);  // (the lanes past the end repeat the last 16 bytes)
+            for (int k0 = 0; k0 < K; k0 += 4) {
+                uint4 w[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int pk = __builtin_amdgcn_readlane(par, min(k0 + u, K - 1) * stride);
+                    w[u] = src[(pk >= 0 ? pk : 0) * (R / 4) + c];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (k0 + u < K) dst[(k0 + u) * (R / 4) + c] = w[u];
+            }
+        }
+        wave_sync();
+        cur ^= 1;
+        if (grows) {
+            tokens(k)[at] = v;
+            add(token_sig(k), v);
+            if (gram) add(gram_sig(k), static_cast<int>(gh));
+        }
+        wave_sync();
+    }
+};
+
+// The steps of a decode of at most kGridBeams beams, the candidates in a
+// grid: lane (k, j) = k J + j holds entry j of beam k's shortlist (J = K
+// unconstrained, where only the first K of a list can be selected; as many
+// as 64 lanes hold with constraints) and every lane of beam k its state, so that a step moves nothing between lanes but the
 // candidates' keys and the selection, through LDS:
 //   * the lane's entry and its row's RowInfo, loaded kGridAhead steps ahead
 //     (three words; a step's chain is shorter than a load's latency);
@@ -1628,9 +1743,17 @@ __device__ __forceinline__ void issue_tagged(const DecodeParams& p, int b, int t
 // operations before them and leaves the later steps' in flight. Bound by the
 // chain of LDS round trips and lane operations, 1.3 us a step: 8 x 32 x 4 x
 // 32000 f32 42 us (the general step, 3.1 us: 97).
+//
+// CON: an entry whose token the beam's signature may hold is looked up in the
+// prefix by the whole wavefront, a beam whose last (n - 1)-gram may have
+// occurred lists its blocked tokens, and a row's entries from J on are left
+// out like those of the list's end: the last one held bounds them.
 // Returns the first step not taken: steps_b, or a step whose rows need a
 // full read or whose words never came (gave_up). s: 64 keys of 16 bytes, then
 // the selection (kGridBeams of 16 bytes, over the shortlists).
+template <bool CON>
+__device__ __forceinline__ int grid_entries(int K) { return CON ? 64 / K : K; }
+
 struct GridState {
     float raw;
     int len, last, ended;
@@ -1641,14 +1764,17 @@ struct GridWords {
     uint32_t i0, i1, i2, i3;  // the row's RowInfo (tags in i1 and i3)
 };
 
-template <bool LOGITS>
+template <bool LOGITS, bool CON>
 __device__ __forceinline__ int grid_steps(const DecodeParams& p, int b, int t, int steps_b, int Kb, int eos_b,
-                                          GridState& g, uint4* s_key, const float* s_pen, const float* s_inv,
-                                          int pen_len, int lane, bool& any_invalid, int& first_bad, bool& gave_up) {
+                                          GridState& g, Prefixes& pre, uint4* s_key, const float* s_pen,
+                                          const float* s_inv, int pen_len, int lane, bool& any_invalid, int& first_bad,
+                                          bool& gave_up) {
     const int K = p.K, T = p.T, M = p.M;
-    const int k = lane / K, j = lane - k * K;
-    const bool on = k < K;  // (K * K lanes of the grid)
-    const int kc = on ? k : 0, jc = on ? j : 0;
+    const int J = grid_entries<CON>(K);
+    const int k = lane / J, j = lane - k * J;
+    const bool on = k < K;  // (K J lanes of the grid)
+    const int kc = on ? k : 0, jc = on ? min(j, M - 1) : 0;
+    constexpr int AHEAD = CON ? kGridAheadCon : kGridAhead;
     const bool coherent = p.step_done != nullptr;
     uint2* const s_key2 = reinterpret_cast<uint2*>(s_key);
     uint4* const s_sel = s_key + 64;
@@ -1665,7 +1791,7 @@ __device__ __forceinline__ int grid_steps(const DecodeParams& p, int b, int t, i
                                  v_score = view(p.scores, 4), v_raw = view(p.raw_scores, 4),
                                  v_flp = view(p.from_logprob, 1), v_lse = view(LOGITS ? p.row_lse : nullptr, 4);
 
-    GridWords ring[kGridAhead];
+    GridWords ring[AHEAD];
     auto issue = [&](GridWords& w, int tn) __attribute__((always_inline)) {
         const int64_t row = ex + static_cast<int64_t>(tn < steps_b ? tn : steps_b - 1) * K + kc;
         const uint32_t* e = reinterpret_cast<const uint32_t*>(p.shortlist + row * M + jc);
@@ -1691,7 +1817,7 @@ __device__ __forceinline__ int grid_steps(const DecodeParams& p, int b, int t, i
         const bool carried = live && eos_b >= 0 && g.ended != 0;
         const bool read = live && !carried;
         uint32_t lpw = w.lp, tokw = w.tok, i0 = w.i0, i1 = w.i1, i2 = w.i2, i3 = w.i3;
-        issue(w, tt + kGridAhead);
+        issue(w, tt + AHEAD);
         if (coherent) {
             // words not yet written (tag 0) are waited for
             const bool miss_info = read && (i1 == 0u || i3 == 0u);
@@ -1719,12 +1845,54 @@ __device__ __forceinline__ int grid_steps(const DecodeParams& p, int b, int t, i
         const uint64_t bad_m = __builtin_amdgcn_ballot_w64(read && i3 != 0u);
         const float inv = (tt + 1 < pen_len) ? s_inv[tt + 1] : 1.0f / length_penalty(tt + 1, p.alpha);
         // the lane's candidate
-        float raw = g.raw + bits_f32(lpw);
-        float score = raw * inv;
+        const float lp = bits_f32(lpw);
+        float raw = g.raw + lp;
         int token = static_cast<int>(tokw);
         bool have = read && j < cnt;
-        const float tau = wave_max_dpp(have && j == K - 1 ? raw : -kInf);
-        have = have && !(raw < tau);
+        uint32_t tail = 0u;
+        if constexpr (CON) {
+            // (a read beam's prefix holds tt tokens)
+            const int n = p.ngram;
+            bool need = false;
+            if (n > 1 && tt >= n - 1) {
+                tail = pre.tail_hash(kc, tt, n);
+                need = tt >= n && read && pre.maybe(pre.gram_sig(kc), static_cast<int>(tail));
+            }
+            int nb = 0;
+            if (__builtin_amdgcn_ballot_w64(need) != 0) {
+                if (on && j == 0) {
+                    pre.plen[k] = need ? tt : -1;
+                    pre.nblk[k] = 0;
+                }
+                wave_sync();
+                pre.list_blocked(n, tt, lane);
+                wave_sync();
+                if (on) nb = pre.nblk[kc];
+                if (have && nb > 0 && in_list(pre.blk + kc * pre.P, nb, token)) have = false;
+            }
+            // tau: K of a row's first K + nb entries are not blocked, each
+            // worth at least its log-prob less the penalty
+            const float tau = wave_max_dpp(read && j < cnt && j == K - 1 + nb ? (p.penalise ? g.raw + (lp - p.log_rep) : raw) : -kInf);
+            have = have && !(raw < tau);
+            if (p.penalise) {
+                uint64_t hits = __builtin_amdgcn_ballot_w64(have && pre.maybe(pre.token_sig(kc), token));
+                uint64_t in = 0;
+                while (hits != 0) {  // (its latency: one round of LDS reads a hit, up to 64 tokens each)
+                    const int l = __ffsll(static_cast<long long>(hits)) - 1;
+                    hits &= hits - 1;
+                    const int v = __builtin_amdgcn_readlane(token, l);
+                    const int32_t* a = pre.tokens(__builtin_amdgcn_readlane(kc, l));
+                    bool found = false;
+                    for (int c0 = 0; c0 < tt; c0 += 64) found = found || a[min(c0 + lane, tt - 1)] == v;
+                    if (__builtin_amdgcn_ballot_w64(found) != 0) in |= 1ull << l;
+                }
+                if ((in >> lane) & 1ull) raw = g.raw + (lp - p.log_rep);
+            }
+        } else {
+            const float tau = wave_max_dpp(have && j == K - 1 ? raw : -kInf);
+            have = have && !(raw < tau);
+        }
+        float score = raw * inv;
         const uint64_t carried_m = __builtin_amdgcn_ballot_w64(carried);
         if (carried_m != 0) {
             const int l = g.len > 1 ? g.len : 1;
@@ -1777,13 +1945,15 @@ __device__ __forceinline__ int grid_steps(const DecodeParams& p, int b, int t, i
         wave_sync();
         const uint4 mine = s_sel[kc];
         const uint4 kth = s_sel[Kb - 1];
-        // Exactness: every candidate left out of a row's list (its entries
-        // from K on too: K others of the row come first) has raw <= fl(p +
-        // bound); the row passes when the Kb-th selected candidate ranks
-        // strictly before that bound's score and raw.
+        // Exactness: every candidate left out of a row's list (unconstrained,
+        // its entries from K on too: K others of the row come first; else
+        // those past the last one held) has raw <= fl(p + bound); the row
+        // passes when the Kb-th selected candidate ranks strictly before that
+        // bound's score and raw.
         bool fail = read && cnt < 0;
-        if (read && bound > -kInf) {
-            const float X = g.raw + bound;
+        const float left = CON && j == J - 1 && cnt > J && lp > bound ? lp : bound;
+        if (read && left > -kInf) {
+            const float X = g.raw + left;
             const float SX = X * inv;
             const float ks = nsel >= Kb ? bits_f32(kth.x) : -kInf, kr = nsel >= Kb ? bits_f32(kth.y) : -kInf;
             fail = fail || (X > -kInf && !((ks > SX) || (ks == SX && kr > X)));
@@ -1791,7 +1961,7 @@ __device__ __forceinline__ int grid_steps(const DecodeParams& p, int b, int t, i
         if (__builtin_amdgcn_ballot_w64(fail) != 0) return false;
         if (bad_m != 0) {
             any_invalid = true;
-            const int at = tt * K + (__ffsll(static_cast<long long>(bad_m)) - 1) / K;  // steps in order, beams in order
+            const int at = tt * K + (__ffsll(static_cast<long long>(bad_m)) - 1) / J;  // steps in order, beams in order
             first_bad = at < first_bad ? at : first_bad;
         }
         const bool sel = on && k < nsel;
@@ -1809,6 +1979,11 @@ __device__ __forceinline__ int grid_steps(const DecodeParams& p, int b, int t, i
         __builtin_amdgcn_raw_buffer_store_b8(static_cast<uint8_t>(flp), v_flp, at / 4, 0, 0);
         if constexpr (LOGITS)
             __builtin_amdgcn_raw_buffer_store_b32(f32_bits(lse), v_lse, read ? at : trace_bytes, 0, 0);
+        if constexpr (CON) {
+            const uint32_t gh = static_cast<uint32_t>(__shfl(static_cast<int>(tail), (parent >= 0 ? parent : 0) * J));
+            pre.advance(parent, tt, lane, J, kc, head && flp != 0, tok, tt, p.ngram > 1 && tt >= p.ngram - 1, gh,
+                        p.ngram > 1);
+        }
         g.raw = rw;
         g.len = length;
         g.last = tok;
@@ -1817,10 +1992,10 @@ __device__ __forceinline__ int grid_steps(const DecodeParams& p, int b, int t, i
         return true;
     };
 #pragma unroll
-    for (int u = 0; u < kGridAhead; ++u) issue(ring[u], t + u);
+    for (int u = 0; u < AHEAD; ++u) issue(ring[u], t + u);
     for (;;) {
 #pragma unroll
-        for (int u = 0; u < kGridAhead; ++u) {
+        for (int u = 0; u < AHEAD; ++u) {
             if (t >= steps_b) return t;
             if (!step(ring[u], t)) return t;
             ++t;
@@ -1849,23 +2024,20 @@ __device__ __forceinline__ void narrow_example(const DecodeParams& p, int pen_le
     Cand* s_cand = reinterpret_cast<Cand*>(smem + 1024 + sizeof(ShortEntry) * static_cast<size_t>(K) * M);  // [64]
     float* s_pen = reinterpret_cast<float*>(s_cand + 64);  // [pen_len]
     float* s_inv = s_pen + pen_len;                        // [pen_len]
-    // Constraints (n-gram blocking, repetition penalty): the beams' prefixes,
-    // signatures of their tokens and of their (n - 1)-grams but the last (two
-    // buffers each: the step's and the next), each read beam's
-    // n-gram-blocked tokens, and per beam its read state and next prefix.
-    const int P = p.prefix_cap, P4 = (P + 3) & ~3, W = sig_words;  // prefix rows P4 words apart (16-byte aligned)
-    uint32_t* s_sig = reinterpret_cast<uint32_t*>(
+    // Constraints (n-gram blocking, repetition penalty): the beams' prefixes
+    Prefixes pre;
+    pre.K = K;
+    pre.P = p.prefix_cap;
+    pre.W = sig_words;
+    pre.R = 2 * sig_words + ((p.prefix_cap + 3) & ~3);
+    pre.shift = 32 - (31 - __builtin_clz(32 * static_cast<uint32_t>(sig_words > 0 ? sig_words : 1)));
+    pre.cur = 0;
+    pre.rec = reinterpret_cast<uint32_t*>(
         smem + ((1024 + sizeof(ShortEntry) * static_cast<size_t>(K) * M + sizeof(Cand) * 64 +
-                 2 * sizeof(float) * static_cast<size_t>(pen_len) + 15) & ~static_cast<size_t>(15)));  // [2][K][W]
-    uint32_t* s_gsig = s_sig + 2 * K * W;                             // [2][K][W]
-    int32_t* s_pre = reinterpret_cast<int32_t*>(s_gsig + 2 * K * W);  // [2][K][P4]
-    int32_t* s_blk = s_pre + 2 * K * P4;                             // [K][P]
-    int32_t* s_nblk = s_blk + K * P;                                 // [K]
-    int32_t* s_plen = s_nblk + K;                                    // [K] prefix length of a read beam, else -1
-    int4* s_next = reinterpret_cast<int4*>(((reinterpret_cast<uintptr_t>(s_plen + K)) + 15) & ~static_cast<uintptr_t>(15));  // [K]
-    uint32_t* s_gnew = reinterpret_cast<uint32_t*>(s_next + K);  // [K] the (n - 1)-gram a new beam's signature takes
-    const int sig_shift = 32 - (31 - __builtin_clz(32 * static_cast<uint32_t>(W > 0 ? W : 1)));
-    int cur = 0;  // the step's prefix buffer
+                 2 * sizeof(float) * static_cast<size_t>(pen_len) + 15) & ~static_cast<size_t>(15)));
+    pre.blk = reinterpret_cast<int32_t*>(pre.rec + 2 * K * pre.R);
+    pre.nblk = pre.blk + K * pre.P;
+    pre.plen = pre.nblk + K;
     for (int l = lane; l < pen_len; l += 64) {
         const float pl = length_penalty(l, p.alpha);
         s_pen[l] = pl;
@@ -1908,11 +2080,11 @@ __device__ __forceinline__ void narrow_example(const DecodeParams& p, int pen_le
         if (lane + 192 < n4) pf3 = src4[lane + 192];
     };
     bool have_pf = false;
-    // Unconstrained decodes of at most kGridBeams beams: their steps go
-    // through grid_steps below, and only those that fail its exactness check
-    // (and the padding steps) through the general step. (The test knob for
-    // waits that give up forces the general step's counted wait.)
-    const bool grid = !CON && K <= kGridBeams && M >= K && p.wait_extra == 0;
+    // Decodes of at most kGridBeams beams: their steps go through grid_steps
+    // below, and only those that fail its exactness check (and the padding
+    // steps) through the general step. (The test knob for waits that give up
+    // forces the general step's counted wait.)
+    const bool grid = K <= kGridBeams && M >= K && p.wait_extra == 0;
     if constexpr (PF) {
         have_pf = steps_b > 0 && !grid;
         if (have_pf) prefetch(0);
@@ -1948,45 +2120,40 @@ __device__ __forceinline__ void narrow_example(const DecodeParams& p, int pen_le
     // the value of token v's log-prob lp in beam k's row (make_cand's rules:
     // false when n-gram blocking removes it, the penalty when it repeats).
     auto in_pre = [&](int k, int lk, int v) -> bool {
-        const uint32_t* sg = s_sig + (cur * K + k) * W;
-        const uint32_t h0 = sig_bit0(v, sig_shift), h1 = sig_bit1(v, sig_shift);
-        if ((((sg[h0 >> 5] >> (h0 & 31u)) & (sg[h1 >> 5] >> (h1 & 31u))) & 1u) == 0u) return false;
-        return in_list(s_pre + (cur * K + k) * P4, lk, v);
+        return pre.maybe(pre.token_sig(k), v) && in_list(pre.tokens(k), lk, v);
     };
     auto constrain = [&](int k, int lk, int nbk, int v, float lp, float& val) -> bool {
-        if (p.ngram > 1 && in_list(s_blk + k * P, nbk, v)) return false;
+        if (p.ngram > 1 && in_list(pre.blk + k * pre.P, nbk, v)) return false;
         val = (p.penalise && in_pre(k, lk, v)) ? lp - p.log_rep : lp;
         return true;
     };
     if constexpr (CON) {
-        for (int i = lane; i < K * W; i += 64) {  // every prefix starts empty
-            s_sig[i] = 0u;
-            s_gsig[i] = 0u;
-        }
+        // every prefix starts empty
+        for (int k = 0; k < K; ++k)
+            for (int i = lane; i < 2 * pre.W; i += 64) pre.gram_sig(k)[i] = 0u;
     }
     // A beam's last n - 1 tokens (its tail), hashed (FNV-1a over the tokens),
     // when it has them: the n-gram list is built only where the tail occurred
     // before, and the tail joins the signature when the beam grows.
     uint32_t tail_h = 0u;
     bool tail_v = false;
-    const int gk = lane / K < K ? lane / K : 0;  // the beam of this lane in grid_steps
+    const int gJ = grid_entries<CON>(K);
+    const int gk = lane / gJ < K ? lane / gJ : 0;  // the beam of this lane in grid_steps
     wave_sync();
 
     for (int t = 0; t < T; ++t) {
-        if constexpr (!CON) {
-            if (grid && t < steps_b && !gave_up) {
-                GridState g{__shfl(raw, gk), __shfl(len, gk), __shfl(last, gk), __shfl(ended ? 1 : 0, gk)};
-                t = grid_steps<LOGITS>(p, b, t, steps_b, Kb, eos_b, g, s_key, s_pen, s_inv, pen_len, lane, any_invalid,
-                                       first_bad, gave_up);
-                const int src = lane < K ? lane * K : 0;
-                const float raw_k = __shfl(g.raw, src);  // (every lane shuffles)
-                const int ended_k = __shfl(g.ended, src);
-                len = __shfl(g.len, src);
-                last = __shfl(g.last, src);
-                raw = beam ? raw_k : -kInf;
-                ended = beam && ended_k != 0;
-                if (t >= T) break;
-            }
+        if (grid && t < steps_b && !gave_up) {
+            GridState g{__shfl(raw, gk), __shfl(len, gk), __shfl(last, gk), __shfl(ended ? 1 : 0, gk)};
+            t = grid_steps<LOGITS, CON>(p, b, t, steps_b, Kb, eos_b, g, pre, s_key, s_pen, s_inv, pen_len, lane,
+                                        any_invalid, first_bad, gave_up);
+            const int src = lane < K ? lane * gJ : 0;
+            const float raw_k = __shfl(g.raw, src);  // (every lane shuffles)
+            const int ended_k = __shfl(g.ended, src);
+            len = __shfl(g.len, src);
+            last = __shfl(g.last, src);
+            raw = beam ? raw_k : -kInf;
+            ended = beam && ended_k != 0;
+            if (t >= T) break;
         }
         const int64_t trace0 = (static_cast<int64_t>(b) * T + t) * K;
         bool pad = t >= steps_b || gave_up;
@@ -2176,64 +2343,21 @@ __device__ __forceinline__ void narrow_example(const DecodeParams& p, int pen_le
                 // the prefix (the signature of those; a hit is checked in full)
                 const int n = p.ngram;
                 tail_v = read && len >= n - 1;
-                tail_h = 0x811C9DC5u;
+                tail_h = 0u;
                 if (tail_v) {
-                    const int32_t* pre = s_pre + (cur * K + lane) * P4;
-                    for (int q = len - (n - 1); q < len; ++q)
-                        tail_h = (tail_h ^ static_cast<uint32_t>(pre[q])) * 0x01000193u;
-                    if (len >= n) {
-                        const uint32_t* gs = s_gsig + (cur * K + lane) * W;
-                        const uint32_t h0 = sig_bit0(static_cast<int>(tail_h), sig_shift);
-                        const uint32_t h1 = sig_bit1(static_cast<int>(tail_h), sig_shift);
-                        need = (((gs[h0 >> 5] >> (h0 & 31u)) & (gs[h1 >> 5] >> (h1 & 31u))) & 1u) != 0u;
-                    }
+                    tail_h = pre.tail_hash(lane, len, n);
+                    need = len >= n && pre.maybe(pre.gram_sig(lane), static_cast<int>(tail_h));
                 }
             }
-            if (beam) s_plen[lane] = need ? len : -1;
             if (__builtin_amdgcn_ballot_w64(need) != 0) {
-                if (beam) s_nblk[lane] = 0;
-                wave_sync();
-                // item = (beam k, position i); eight items per lane a round,
-                // every read of a round in flight together
-                // (beam k's positions at a power-of-two stride 2^ps >= t: no
-                // division)
-                const int n = p.ngram, Pt = min(P, t);
-                const int ps = Pt > 1 ? 32 - __builtin_clz(static_cast<uint32_t>(Pt - 1)) : 0, total = K << ps;
-                for (int j0 = 0; j0 < total; j0 += 8 * 64) {
-                    int kk[8], ii[8], tl[8];
-                    bool on[8];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) {
-                        const int j = j0 + 64 * u + lane;
-                        const int jc = j < total ? j : 0;
-                        kk[u] = jc >> ps;
-                        ii[u] = jc & ((1 << ps) - 1);
-                        const int Lk = s_plen[kk[u]];
-                        on[u] = j < total && ii[u] + n <= Lk;  // (a beam not read: -1)
-                        tl[u] = on[u] ? Lk - (n - 1) : 0;
-                    }
-                    bool same[8] = {true, true, true, true, true, true, true, true};
-                    for (int q = 0; q < n - 1; ++q) {
-                        int32_t a[8], c[8];
-#pragma unroll
-                        for (int u = 0; u < 8; ++u) {
-                            const int32_t* pre = s_pre + (cur * K + kk[u]) * P4;
-                            a[u] = pre[on[u] ? ii[u] + q : 0];
-                            c[u] = pre[tl[u] + q];
-                        }
-#pragma unroll
-                        for (int u = 0; u < 8; ++u) same[u] = same[u] && a[u] == c[u];
-                    }
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) {
-                        if (on[u] && same[u]) {
-                            const int slot = atomicAdd(&s_nblk[kk[u]], 1);
-                            s_blk[kk[u] * P + slot] = s_pre[(cur * K + kk[u]) * P4 + ii[u] + n - 1];
-                        }
-                    }
+                if (beam) {
+                    pre.plen[lane] = need ? len : -1;
+                    pre.nblk[lane] = 0;
                 }
                 wave_sync();
-                nblk = beam ? s_nblk[lane] : 0;
+                pre.list_blocked(p.ngram, t, lane);
+                wave_sync();
+                nblk = beam ? pre.nblk[lane] : 0;
             }
         }
 
@@ -2480,82 +2604,13 @@ __device__ __forceinline__ void narrow_example(const DecodeParams& p, int pen_le
             pend_c = c;
         }
         if constexpr (CON) {
-            // each selected beam: its parent's prefix, then its token, and the
-            // signature of both, into the other buffer
+            // each selected beam: its parent's prefix and signatures, then its token
             const int par = c.parent;
             const int len_par = __shfl(len, par >= 0 ? par : 0);
             const uint32_t gh_par = static_cast<uint32_t>(__shfl(static_cast<int>(tail_h), par >= 0 ? par : 0));
             const int gv_par = __shfl(tail_v ? 1 : 0, par >= 0 ? par : 0);
-            const bool grows = par >= 0 && c.flp && c.token >= 0;
-            if (beam) {
-                s_next[lane] = make_int4(par, grows ? c.token : -1, par >= 0 ? len_par : 0, grows && gv_par ? 1 : 0);
-                s_gnew[lane] = gh_par;
-            }
-            wave_sync();
-            const int nxt = cur ^ 1;
-            const int Lc = min(P, t + 1);  // the new prefixes' length, at most
-            // 16 bytes an item: the parent's prefix (its appended token's
-            // word is written over after), then its signature with the
-            // token's two bits; four items per lane a round, their reads in
-            // flight together
-            // (each beam's chunks at power-of-two strides: no division)
-            const int C4 = (Lc + 3) >> 2, W4 = W / 4;
-            const int cs = C4 > 1 ? 32 - __builtin_clz(static_cast<uint32_t>(C4 - 1)) : 0;
-            const int ws = 31 - __builtin_clz(static_cast<uint32_t>(W4));
-            // the (n - 1)-gram signatures follow the token signatures
-            const int ns = K << ws, np = K << cs, total = np + (p.ngram > 1 ? 2 : 1) * ns;
-            uint4* const s_pre4 = reinterpret_cast<uint4*>(s_pre);
-            uint4* const s_sig4 = reinterpret_cast<uint4*>(s_sig);
-            for (int j0 = 0; j0 < total; j0 += 5 * 64) {
-                int dst[5];
-                bool isp[5];
-                uint4 v[5];
-#pragma unroll
-                for (int u = 0; u < 5; ++u) {
-                    const int j = j0 + 64 * u + lane;
-                    const int jc = j < total ? j : 0;
-                    isp[u] = jc < np;
-                    const bool isg = jc >= np + ns;  // an (n - 1)-gram signature chunk
-                    const int jj = isp[u] ? jc : jc - np - (isg ? ns : 0), sh = isp[u] ? cs : ws;
-                    const int k = jj >> sh, q = jj & ((1 << sh) - 1);
-                    const int4 nx = s_next[k];
-                    const int pk = nx.x >= 0 ? nx.x : 0;
-                    if (isp[u]) {
-                        dst[u] = j < total && nx.x >= 0 && q < C4 ? ((nxt * K + k) * P4 >> 2) + q : -1;
-                        v[u] = s_pre4[((cur * K + pk) * P4 >> 2) + (q < C4 ? q : 0)];
-                    } else {
-                        // (s_gsig is s_sig + 2 K W words: the same buffers, 2 K W4 chunks on)
-                        const int g4 = isg ? 2 * K * W4 : 0;
-                        dst[u] = j < total ? g4 + (nxt * K + k) * W4 + q : -1;
-                        v[u] = s_sig4[g4 + (cur * K + pk) * W4 + q];
-                        if (nx.x < 0) v[u] = make_uint4(0u, 0u, 0u, 0u);
-                        const bool add = isg ? nx.w != 0 : nx.x >= 0 && nx.y >= 0;
-                        if (add) {
-                            const int hv = isg ? static_cast<int>(s_gnew[k]) : nx.y;
-                            const uint32_t hs[2] = {sig_bit0(hv, sig_shift), sig_bit1(hv, sig_shift)};
-#pragma unroll
-                            for (int h2 = 0; h2 < 2; ++h2) {
-                                const uint32_t h = hs[h2];
-                                if (static_cast<int>(h >> 7) != q) continue;
-                                const uint32_t m = 1u << (h & 31u);
-                                switch ((h >> 5) & 3u) {
-                                    case 0: v[u].x |= m; break;
-                                    case 1: v[u].y |= m; break;
-                                    case 2: v[u].z |= m; break;
-                                    default: v[u].w |= m; break;
-                                }
-                            }
-                        }
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < 5; ++u)
-                    if (dst[u] >= 0) (isp[u] ? s_pre4 : s_sig4)[dst[u]] = v[u];
-            }
-            wave_sync();
-            if (beam && par >= 0 && c.flp && c.token >= 0) s_pre[(nxt * K + lane) * P4 + len_par] = c.token;
-            wave_sync();
-            cur = nxt;
+            const bool grows = beam && par >= 0 && c.flp && c.token >= 0;
+            pre.advance(par, t, lane, 1, lane, grows, c.token, len_par, gv_par != 0, gh_par, p.ngram > 1);
         }
         const int parent_ended = __shfl(ended ? 1 : 0, c.parent >= 0 ? c.parent : 0);
         ended = c.parent >= 0 && (parent_ended != 0 || is_eos_of(p, b, c.token));

@@ -31,6 +31,7 @@ constexpr int kWideRank = 4;  // candidates per thread of the rank compaction be
 constexpr int kNarrowMaxK = 16;       // the running list lives in one 16-lane DPP row
 constexpr int kGridBeams = 8;         // beams whose K * K candidates fit one wavefront's lanes (grid_steps)
 constexpr int kGridAhead = 4;         // steps its words are loaded ahead
+constexpr int kGridAheadCon = 2;      // with constraints (longer steps, and twice the step's code instead of four times)
 constexpr int kNarrowPf = 4;          // 16-byte prefetch registers per lane (K * M <= 512)
 constexpr int kNarrowPenCap = 1024;   // lengths with a penalty in LDS (larger ones are computed)
 constexpr int kNarrowRescanUnroll = 16;
@@ -69,7 +70,6 @@ inline size_t narrow_wave_bytes(const DecodeParams& p, int W) {
     if (p.constrained) {
         const size_t P4 = (P + 3) & ~static_cast<size_t>(3);
         n += sizeof(uint32_t) * 4 * K * static_cast<size_t>(W) + sizeof(int32_t) * (2 * K * P4 + K * P + 2 * K);
-        n = ((n + 15) & ~static_cast<size_t>(15)) + sizeof(int4) * K + sizeof(uint32_t) * K;
     }
     return (n + 15) & ~static_cast<size_t>(15);
 }
