@@ -128,6 +128,62 @@ __device__ __forceinline__ uint32_t key_pattern(int key) {
     return static_cast<uint16_t>(key < 0 ? (key ^ 0x7fff) : key);
 }
 
+// max(a, b, c) (a NaN operand may lose the others: only rows without NaN use it).
+__device__ __forceinline__ float max3(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
+// Thread maximum, NaN / +inf flags of 16-byte blocks: 1.5 operations an element.
+template <int DT>
+struct Extremes {
+    float fmax = -kInf;                   // float32
+    uint32_t smax, smin = 0x7fff7fffu, umax = 0u;  // bit patterns (16-bit: packed)
+
+    __device__ __forceinline__ Extremes() : smax(DT == 0 ? 0x80000000u : 0x80008000u) {}
+
+    __device__ __forceinline__ void take(const v4u32& d) {
+        if constexpr (DT == 0) {
+            fmax = max3(fmax, bits_f32(d.x), bits_f32(d.y));
+            fmax = max3(fmax, bits_f32(d.z), bits_f32(d.w));
+            auto imax = [](uint32_t a, uint32_t b) { return static_cast<int>(a) > static_cast<int>(b) ? a : b; };
+            auto vmax = [](uint32_t a, uint32_t b) { return a > b ? a : b; };
+            smax = imax(imax(smax, d.x), d.y);
+            smax = imax(imax(smax, d.z), d.w);
+            umax = vmax(vmax(umax, d.x), d.y);
+            umax = vmax(vmax(umax, d.z), d.w);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                smax = pk_max_i16(smax, d[i]);
+                smin = pk_min_i16(smin, d[i]);
+                umax = pk_max_u16(umax, d[i]);
+            }
+        }
+    }
+    // The maximum (of a thread without NaN / +inf) and whether there was one.
+    __device__ __forceinline__ float result(bool& bad) const {
+        if constexpr (DT == 0) {
+            bad = static_cast<int>(smax) >= 0x7f800000 || umax > 0xff800000u;
+            return fmax;
+        } else {
+            const int pos_inf = DT == 1 ? 0x7c00 : 0x7f80;
+            const uint32_t neg_inf = DT == 1 ? 0xfc00u : 0xff80u;
+            bad = false;
+            int best = -32768;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int16_t hmax = static_cast<int16_t>(smax >> (16 * h));
+                const int16_t hmin = static_cast<int16_t>(smin >> (16 * h));
+                bad = bad || hmax >= pos_inf || ((umax >> (16 * h)) & 0xffffu) > neg_inf;
+                best = max(best, key16(static_cast<uint16_t>(hmax >= 0 ? hmax : hmin)));
+            }
+            return pattern_value<DT>(key_pattern(best));
+        }
+    }
+};
+
 // The maximum over a wavefront's 64 lanes (every lane gets it).
 __device__ __forceinline__ int wave_max_int(int x) {
     const int lo = static_cast<int>(0x80000000u);

@@ -28,6 +28,12 @@
 //     registers; each survivor's rank among them (a count of the survivors
 //     before it) places it in the shortlist, every thread ranking some.
 //
+// Bound by its loads and, between a row's last load and the next row's first,
+// by the passes over the registers: with the maximum and the flag at 1.5
+// operations an element, the block test at one and the edge test left out of
+// whole blocks, 16 x 64 x 4 x 50000 f32 152 -> 144 us (5.6 TB/s), 8 x 32 x 4 x
+// 32000 35 -> 32; 16-bit rows of 50257 613 -> 607.
+//
 // A row with NaN or +inf keeps no shortlist (the select pass reads such a row
 // in full), as in the other row passes.
 #include <hip/hip_runtime.h>
@@ -120,6 +126,40 @@ __device__ __forceinline__ void next_row_options(const DecodeParams& p, int64_t 
     }
 }
 
+// The pattern of a value taken from a 16-bit element.
+template <int DT>
+__device__ __forceinline__ uint32_t pattern_of(float x) {
+    if constexpr (DT == 1) return __builtin_bit_cast(uint16_t, static_cast<_Float16>(x));
+    else return f32_bits(x) >> 16;
+}
+
+// Whether a block without NaN / +inf holds an element >= theta. 16-bit
+// elements by their patterns, two an operation: theta <= 0 (log-probs), where
+// the smallest unsigned pattern is at most theta's (or any is non-negative);
+// else where the largest signed one is at least theta's.
+template <int DT>
+struct Reach {
+    float theta;
+    bool pos;
+    int pat;
+    __device__ __forceinline__ explicit Reach(float th)
+        : theta(bits_f32(__builtin_amdgcn_readfirstlane(f32_bits(th)))), pos(theta > 0.0f), pat(0) {
+        if constexpr (DT != 0) pat = static_cast<int>(theta == 0.0f ? 0x8000u : pattern_of<DT>(theta));
+    }
+    __device__ __forceinline__ bool operator()(const v4u32& d) const {
+        if constexpr (DT == 0) {
+            const float m = max3(bits_f32(d.x), bits_f32(d.y), bits_f32(d.z));
+            return max3(m, m, bits_f32(d.w)) >= theta;
+        } else if (pos) {
+            const uint32_t m = pk_max_i16(pk_max_i16(d.x, d.y), pk_max_i16(d.z, d.w));
+            return max(static_cast<int>(static_cast<int16_t>(m)), static_cast<int>(m) >> 16) >= pat;
+        } else {
+            const uint32_t m = pk_min_u16(pk_min_u16(d.x, d.y), pk_min_u16(d.z, d.w));
+            return static_cast<int>(min(m & 0xffffu, m >> 16)) <= pat;
+        }
+    }
+};
+
 // Persistent: a workgroup takes rows in turn (tickets in the overlapped
 // decode, else its own stride), and issues the loads of its next row as soon
 // as the current row's blocks that can hold survivors are copied to LDS, so
@@ -174,9 +214,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(C <= 32 && N
 
     while (r < rows) {
 
-        // Elements outside the row become -inf.
+        // Elements outside the row become -inf (a wave-uniform test leaves
+        // out the blocks that lie inside it for every thread).
 #pragma unroll
         for (int c = 0; c < C; ++c) {
+            if ((c > 0 || lead_e == 0) && (c + 1) * NT * epb - lead_e <= V) continue;
             const int v0 = (c * NT + tid) * epb - lead_e;
             if (v0 < 0 || v0 + epb > V) {
 #pragma unroll
@@ -185,49 +227,16 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(C <= 32 && N
             }
         }
 
-        // Thread maximum over x < +inf, its order key, and the NaN / +inf flag.
-        float tmax = -kInf;
+        // Thread maximum and the NaN / +inf flag (the maximum counts only
+        // where no thread has one), and its order key.
+        Extremes<DT> ex;
+#pragma unroll
+        for (int c = 0; c < C; ++c) ex.take(d[c]);
+        bool bad;
+        const float tmax = ex.result(bad);
         uint32_t tkey;
-        bool bad = false;
-        if constexpr (DT == 0) {
-#pragma unroll
-            for (int c = 0; c < C; ++c) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float x = bits_f32(d[c][i]);
-                    bad = bad || __builtin_amdgcn_classf(x, 0x203);  // sNaN, qNaN, +inf
-                    tmax = fmaxf(tmax, x);
-                }
-            }
-            tkey = ordered_key(tmax);
-        } else {
-            // Signed max/min and unsigned max of the raw patterns: the largest
-            // value is the largest non-negative pattern, else the smallest
-            // (most negative) signed one; a signed max >= +inf's pattern flags
-            // +inf or a positive NaN, an unsigned max above -inf's a negative NaN.
-            uint32_t smax = 0x80008000u, smin = 0x7fff7fffu, umax = 0u;
-#pragma unroll
-            for (int c = 0; c < C; ++c) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    smax = pk_max_i16(smax, d[c][i]);
-                    smin = pk_min_i16(smin, d[c][i]);
-                    umax = pk_max_u16(umax, d[c][i]);
-                }
-            }
-            const int pos_inf = DT == 1 ? 0x7c00 : 0x7f80;
-            const uint32_t neg_inf = DT == 1 ? 0xfc00u : 0xff80u;
-            int best = -32768;
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int16_t hmax = static_cast<int16_t>(smax >> (16 * h));
-                const int16_t hmin = static_cast<int16_t>(smin >> (16 * h));
-                bad = bad || hmax >= pos_inf || ((umax >> (16 * h)) & 0xffffu) > neg_inf;
-                best = max(best, key16(static_cast<uint16_t>(hmax >= 0 ? hmax : hmin)));
-            }
-            tmax = pattern_value<DT>(key_pattern(best));
-            tkey = static_cast<uint32_t>(best + 32768);  // the signed key, biased to 16 unsigned bits
-        }
+        if constexpr (DT == 0) tkey = ordered_key(tmax);
+        else tkey = static_cast<uint32_t>(key16(pattern_of<DT>(tmax)) + 32768);  // the signed key, biased
         s_tkey[tid] = tkey;
         if (__any(bad) && (tid & 63) == 0) s_bad = 1;
         __syncthreads();
@@ -250,7 +259,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(C <= 32 && N
                 }
                 float th;
                 if constexpr (DT == 0) {
-                    th = key_value(mth_largest_key<32>(k4, M));
+                    th = key_value(mth_largest_key<32, 12>(k4, M));  // (rounded down: still at least M reach it)
                 } else {
                     th = pattern_value<DT>(key_pattern(static_cast<int>(mth_largest_key<16>(k4, M)) - 32768));
                 }
@@ -273,12 +282,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(C <= 32 && N
             // kept in registers from the edge test above)
             int vt = tid * epb - lead_e;
             asm volatile("" : "+v"(vt));
+            const Reach<DT> reach(theta);
 #pragma unroll
             for (int c = 0; c < C; ++c) {
-                float bm = -kInf;
-#pragma unroll
-                for (int i = 0; i < epb; ++i) bm = fmaxf(bm, element_of<DT>(d[c], i));
-                if (bm >= theta) {
+                if (reach(d[c])) {
                     const int slot = atomicAdd(&s_nblk, 1);
                     if (slot < kLpBlockCap) {
                         s_blk[slot] = d[c];
