@@ -40,7 +40,7 @@ HIP_FLAGS = [
 ]
 
 LIB_SOURCES = ["csrc/api.hip", "csrc/host_abi.cpp", "csrc/host_results.cpp", "csrc/decode.hip", "csrc/row_pass.hip",
-               "csrc/row_logprob.hip", "csrc/row_relay.hip", "csrc/row_stream.hip",
+               "csrc/row_logprob.hip", "csrc/row_relay.hip", "csrc/row_stream.hip", "csrc/row_short.hip",
                "csrc/select.hip", "csrc/select_f32.hip",
                "csrc/select_f16.hip", "csrc/select_bf16.hip", "csrc/backward.hip"]
 

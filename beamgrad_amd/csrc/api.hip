@@ -803,7 +803,7 @@ DBS_CUDA_EXPORT int dbs_hip_set_decode_overlap(int on) {
 }
 
 DBS_CUDA_EXPORT int dbs_hip_set_row_pass(int kind) {
-    if (kind < -1 || kind > 7 || kind == 4 || kind == 6) return -2;
+    if (kind < -1 || kind > 8 || kind == 4 || kind == 6) return -2;
     return dbs_hip::g_row_pass_kind.exchange(kind);
 }
 

@@ -203,6 +203,10 @@ bool row_relay_eligible(const DecodeParams& p);
 // its full register capacity, so shorter rows take the stream pass).
 bool row_relay_preferred(const DecodeParams& p);
 hipError_t launch_row_relay(const DecodeParams& p, int64_t rows, hipStream_t stream);
+// Short rows of any type and alignment, a wavefront each (row_short.hip).
+bool row_short_eligible(const DecodeParams& p);
+bool row_short_preferred(const DecodeParams& p);
+hipError_t launch_row_short(const DecodeParams& p, int64_t rows, hipStream_t stream);
 // Rows of any type, size and alignment, read twice (row_stream.hip).
 bool row_stream_eligible(const DecodeParams& p);
 hipError_t launch_row_stream(const DecodeParams& p, int64_t rows, hipStream_t stream);

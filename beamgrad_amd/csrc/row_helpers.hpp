@@ -128,6 +128,50 @@ __device__ __forceinline__ uint32_t key_pattern(int key) {
     return static_cast<uint16_t>(key < 0 ? (key ^ 0x7fff) : key);
 }
 
+// exp_nonpositive(x - m) for every x: the same value bit for bit, with n = m -
+// x, in 24 operations.
+//   * floor(y + 0.5), y = fl(d log2 e) for d = -n in [-87, 0], as the nearest
+//     integer of y (1 - 2^-24) (ties, at negative half-integers y, go up as
+//     the floor takes them), taken by adding 1.5 2^23;
+//   * k 0.693359375 is exact (9 and 7 significant bits), so one fused
+//     operation gives fl(d - fl(k 0.693359375));
+//   * the power of two is added to the exponent: p 2^k is normal for d >= -87;
+//   * 0 unless the pattern of n is at most 87's: n > 87, NaN (a NaN x), +inf
+//     (x = -inf) and -inf (x = +inf) all lie above it as unsigned integers.
+// Checked against the reference's steps for every one of the 2^30 floats d in
+// [-87, 0]: the same k and the same result.
+__device__ __forceinline__ float exp_term(float m, float x) {
+    const float n = m - x;
+    const float y = n * -1.44269504088896341f;
+    const float t = __builtin_fmaf(y, 0.99999994f, 12582912.0f);
+    const float k = t - 12582912.0f;
+    const float r = __builtin_fmaf(k, -0.693359375f, -n) - k * -2.12194440e-4f;
+    const float r2 = r * r;
+    float p = 1.9875691500e-4f;
+    p = p * r + 1.3981999507e-3f;
+    p = p * r + 8.3334519073e-3f;
+    p = p * r + 4.1665795894e-2f;
+    p = p * r + 1.6666665459e-1f;
+    p = p * r + 5.0000001201e-1f;
+    p = (p * r2 + r) + 1.0f;
+    const float e = bits_f32(f32_bits(p) + (f32_bits(t) << 23));
+    return f32_bits(n) <= 0x42ae0000u ? e : 0.0f;
+}
+
+template <int DT>
+__device__ __forceinline__ float raw_value(uint32_t h) {  // an element as loaded
+    if constexpr (DT == 0) return bits_f32(h);
+    else if constexpr (DT == 1) return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(h)));
+    else return bits_f32(h << 16);
+}
+
+// One element of the row at byte offset voff + soff of its view.
+template <int DT>
+__device__ __forceinline__ uint32_t load_raw(__amdgpu_buffer_rsrc_t rs, int voff, int soff) {
+    if constexpr (DT == 0) return __builtin_amdgcn_raw_buffer_load_b32(rs, voff, soff, kRowLoadPolicy);
+    else return static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b16(rs, voff, soff, kRowLoadPolicy));
+}
+
 // max(a, b, c) (a NaN operand may lose the others: only rows without NaN use it).
 __device__ __forceinline__ float max3(float a, float b, float c) {
     float r;

@@ -152,16 +152,18 @@ std::atomic<int> g_row_pass_kind{-1};
 
 namespace {
 
-// The kernel of a row pass. Log-prob rows: the one-read kernel up to its
+// The kernel of a row pass. Rows of up to 6144 entries: the short-row kernel,
+// where there are enough of them. Log-prob rows: the one-read kernel up to its
 // register limit (16 x 64 x 4 x 50000 f32: 345 us on the two-pass kernel, 264
-// on the stream kernel, 152). Logits: the relay kernel for the bfloat16 rows it
+// on the stream kernel, 144). Logits: the relay kernel for the bfloat16 rows it
 // fills. Every other row: the stream kernel (row pass of 16 x 64 x 4 x 50257
-// f32 logits 280 us, 487 on the two-pass kernel; 8 x 32 x 8 x 128256 f16 214,
+// f32 logits 279 us, 487 on the two-pass kernel; 8 x 32 x 8 x 128256 f16 203,
 // 1115; f32 log-prob rows of 128256 307, 708). A forced kind that does not
 // apply, or is no longer a kernel of its own, takes the two-pass kernel.
-enum Kernel { kTwoPass, kLogprob, kRelay, kStream };
+enum Kernel { kTwoPass, kLogprob, kRelay, kStream, kShort };
 Kernel row_kernel(const DecodeParams& p) {
     const int kind = g_row_pass_kind.load(std::memory_order_relaxed);
+    if ((kind == 8 || (kind == -1 && row_short_preferred(p))) && row_short_eligible(p)) return kShort;
     if ((kind == -1 || kind == 3) && row_logprob_eligible(p)) return kLogprob;
     if ((kind == 5 || (kind == -1 && row_relay_preferred(p))) && row_relay_eligible(p)) return kRelay;
     if ((kind == -1 || kind == 7) && row_stream_eligible(p)) return kStream;
@@ -182,6 +184,7 @@ hipError_t launch_row_pass(const DecodeParams& p, hipStream_t stream) {
         case kLogprob: return launch_row_logprob(p, rows, stream);
         case kRelay: return launch_row_relay(p, rows, stream);
         case kStream: return launch_row_stream(p, rows, stream);
+        case kShort: return launch_row_short(p, rows, stream);
         case kTwoPass: break;
     }
     const dim3 grid(static_cast<unsigned>(rows));

@@ -25,7 +25,12 @@
 // (measured: 3.7-4.0 TB/s of rows read twice whatever their number in flight,
 // 7.2 TB/s read once), and binary16 and float32 terms cost 25 vector operations
 // each (exp_term), 28 an element with the first read's: 2.9 TB/s of binary16
-// and 5.8 TB/s of float32 rows at 2.4 GHz. Keeping the row on chip instead
+// and 5.8 TB/s of float32 rows at 2.4 GHz (measured, row bytes over time: 8 x 32
+// x 8 x 128256 f16 203 us, 2.5 TB/s; 16 x 64 x 4 x 50257 f32 279 us, 2.9 TB/s:
+// two reads at 5.9). bfloat16 terms come from a table (7 operations an element
+// and 8192 terms a row), 32 x 48 x 5 x 50257 327 us, 2.4 TB/s. Loading 16-bit
+// rows by dwords (half the loads, lanes exchanged after) was slower, 238 and
+// 337 us. Keeping the row on chip instead
 // pays only where the arithmetic leaves room: long bfloat16 rows (a table of the
 // terms), which the relay pass takes where alignment allows.
 #include <hip/hip_runtime.h>
@@ -45,51 +50,7 @@ constexpr int kStRecords = 432;   // groups holding survivors, at most (else the
 constexpr int kStSurvivors = 432; // survivors, at most (likewise)
 constexpr int kStTableRow = 12000;  // bfloat16 rows from which the term table pays (8192 terms against 5 of 25 operations an element)
 constexpr int kStBlocks = 8;    // 16-byte loads in flight per thread in the first read
-constexpr int kFirstPolicy = 0, kSecondPolicy = 2;  // (the second read streams: 4.0 against 3.7 TB/s)
-
-// exp_nonpositive(x - m) for every x: the same value bit for bit, with n = m -
-// x, in 24 operations.
-//   * floor(y + 0.5), y = fl(d log2 e) for d = -n in [-87, 0], as the nearest
-//     integer of y (1 - 2^-24) (ties, at negative half-integers y, go up as
-//     the floor takes them), taken by adding 1.5 2^23;
-//   * k 0.693359375 is exact (9 and 7 significant bits), so one fused
-//     operation gives fl(d - fl(k 0.693359375));
-//   * the power of two is added to the exponent: p 2^k is normal for d >= -87;
-//   * 0 unless the pattern of n is at most 87's: n > 87, NaN (a NaN x), +inf
-//     (x = -inf) and -inf (x = +inf) all lie above it as unsigned integers.
-// Checked against the reference's steps for every one of the 2^30 floats d in
-// [-87, 0]: the same k and the same result.
-__device__ __forceinline__ float exp_term(float m, float x) {
-    const float n = m - x;
-    const float y = n * -1.44269504088896341f;
-    const float t = __builtin_fmaf(y, 0.99999994f, 12582912.0f);
-    const float k = t - 12582912.0f;
-    const float r = __builtin_fmaf(k, -0.693359375f, -n) - k * -2.12194440e-4f;
-    const float r2 = r * r;
-    float p = 1.9875691500e-4f;
-    p = p * r + 1.3981999507e-3f;
-    p = p * r + 8.3334519073e-3f;
-    p = p * r + 4.1665795894e-2f;
-    p = p * r + 1.6666665459e-1f;
-    p = p * r + 5.0000001201e-1f;
-    p = (p * r2 + r) + 1.0f;
-    const float e = bits_f32(f32_bits(p) + (f32_bits(t) << 23));
-    return f32_bits(n) <= 0x42ae0000u ? e : 0.0f;
-}
-
-template <int DT>
-__device__ __forceinline__ float raw_value(uint32_t h) {  // an element as loaded
-    if constexpr (DT == 0) return bits_f32(h);
-    else if constexpr (DT == 1) return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(h)));
-    else return bits_f32(h << 16);
-}
-
-// One element of the row at byte offset voff + soff of its view.
-template <int DT>
-__device__ __forceinline__ uint32_t load_raw(__amdgpu_buffer_rsrc_t rs, int voff, int soff) {
-    if constexpr (DT == 0) return __builtin_amdgcn_raw_buffer_load_b32(rs, voff, soff, kSecondPolicy);
-    else return static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b16(rs, voff, soff, kSecondPolicy));
-}
+constexpr int kFirstPolicy = 0;  // (the second read streams, kRowLoadPolicy: 4.0 against 3.7 TB/s)
 
 // TABLE: bfloat16 logits rows long enough for the term table.
 template <int DT, bool LOGITS, bool TABLE>

@@ -232,13 +232,13 @@ DBS_CUDA_EXPORT int dbs_hip_profile_read(int kernel, double* total_ms, int64_t* 
 
 /* Row-pass kernel choice for tests and measurements (no counterpart in the
  * reference; every choice gives the same results): -1 automatic (the
- * default: for log-prob rows the one-read log-prob kernel where it applies;
+ * default: the short-row kernel for rows of up to 6144 entries where there are
+ * enough of them; for log-prob rows the one-read log-prob kernel where it applies;
  * for logits the relay kernel for the bfloat16 rows it fills; for every other
  * row the stream kernel), 0 two-pass, 3 one-read log-prob rows (any dtype, rows
  * up to 425968 bytes), 5 relay for bfloat16 logits (V % 8 == 0, 16-byte aligned
- * rows, V <= 155648), 7 stream (any dtype and V); 1 and 2 are accepted and
- * take the two-pass kernel; 4 and 6 are not
- * kernels (-2). A kernel that does not apply to a decode falls back to the
+ * rows, V <= 155648), 7 stream (any dtype and V), 8 short rows (V <= 6144); 1 and 2 are accepted and
+ * take the two-pass kernel; 4 and 6 are not kernels (-2). A kernel that does not apply to a decode falls back to the
  * two-pass one. Returns the previous choice, or -2 for an invalid
  * argument. */
 DBS_CUDA_EXPORT int dbs_hip_set_row_pass(int kind);
@@ -246,8 +246,8 @@ DBS_CUDA_EXPORT int dbs_hip_set_row_pass(int kind);
 /* Whether a multi-step decode runs its select pass alongside the row pass, on
  * a second stream that the caller's stream then waits for (no counterpart in
  * the reference; the results are the same either way): -1 automatic (the
- * default: constrained decodes, whose select pass is as long as the row
- * pass), 1 always, 0 never (the select pass after the row pass on the
+ * default: constrained decodes, decodes whose row pass is the relay kernel, and
+ * decodes with the workgroup select pass where it can hold its CUs), 1 always, 0 never (the select pass after the row pass on the
  * caller's stream). Applies when at most half the CUs would be left to the
  * select pass (one per example for the workgroup pass, one per four examples
  * for the one-wavefront pass). Returns the previous setting, or -2 for an
