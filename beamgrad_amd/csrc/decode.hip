@@ -143,8 +143,9 @@ DecodeLayout decode_layout(int B, int T, int K, int V, bool constrained, bool st
     // row: K rows share the K selections, and only the first steps, whose
     // candidates come from a few rows, read rows in full (select_kernel's WIDE;
     // 4 x 8 x 256 x 32000 f32 log-probs: 38.7 ms reading every row in full,
-    // 0.49 ms with the lists, the row pass alone 0.18). Larger relaxed pools rescan every row, and so does a decode whose
-    // caller's workspace has no room for the lists (wide_lists false).
+    // 0.45 ms with the lists, the row pass alone 0.18). Larger relaxed pools
+    // rescan every row, and so does a decode whose caller's workspace has no
+    // room for the lists (wide_lists false).
     const int kept = keep > 0 ? keep : K;
     int M = kept <= 64 ? ((kept + 16 + 7) / 8) * 8 : (kept == K && wide_lists ? 80 : 0);
     if (const char* env = std::getenv("DBS_HIP_SHORTLIST")) {
@@ -327,14 +328,18 @@ size_t sync_bytes(int B, int T) {
 // pass can run alongside on a second stream, following the row pass step by
 // step: the row pass is queued first and never waits on the select pass, and
 // its rows are handed out by ticket, so it always progresses on the CUs left.
-// By default constrained decodes (n-gram blocking, repetition penalty) do,
-// whose select pass is as long as the row pass; decodes whose row pass is
-// one of the persistent kernels (16-bit rows kept on chip), which lose only
-// the CUs they leave free (MI355X: C2 2.00 -> 1.89 ms, C5 forward 2.35 ->
-// 1.75 ms); and decodes with the workgroup select pass beside the one-read
-// log-prob kernel (one workgroup per row) when at most one example per 8 CUs
-// lets the select pass hold its CUs (C4 2.73 -> 2.13 ms; shared CUs made it
-// 3.53 ms).
+// By default constrained decodes (n-gram blocking, repetition penalty) do (64 x
+// 128 x 5 x 50257 f16: 720 us of row pass and 433 of select pass take 837);
+// decodes whose row pass is the relay kernel (one workgroup per CU, the row on
+// chip), which lose only the CUs they leave free (32 x 64 x 8 x 151936 bf16
+// 2.00 -> 1.89 ms, 16 x 128 x 8 x 128256 2.35 -> 1.75); and decodes with the
+// workgroup select pass when at most one example per 8 CUs lets the select
+// pass hold its CUs (16 x 64 x 64 x 32000 f32 2.73 -> 2.13 ms; shared CUs made
+// it 3.53 ms). The one-wavefront pass of an unconstrained decode ends sooner
+// after the stream and log-prob passes than beside them: 40 us of launches and
+// events, and rows that complete several per CU at a time, 100 us behind their
+// step (float32 and float16 logits; batches of 0.5 GB and more of bfloat16 or
+// log-probs would gain 5-15 %).
 // *fault: the overlapped decode's fault word (non-zero once a select-pass
 // wait gave up), else null.
 hipError_t launch_decode(const DecodeParams& p0, const DecodeLayout& L, hipStream_t stream, char* ws,
@@ -364,7 +369,7 @@ hipError_t launch_decode(const DecodeParams& p0, const DecodeLayout& L, hipStrea
     }
     const bool persistent = row_pass_persistent(p);
     const int reserve = select_reserve_cus(p, persistent);
-    // Beside a row pass of one workgroup per row, a select pass of at most
+    // Beside a row pass of several workgroups per CU, a select pass of at most
     // one workgroup per 8 CUs holds its CUs (select_hold: the workgroup pass,
     // and the one-wavefront pass of a constrained decode); a larger one
     // shares them. An unconstrained decode overlaps such a row pass only

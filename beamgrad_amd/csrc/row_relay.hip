@@ -730,7 +730,7 @@ bool row_relay_eligible(const DecodeParams& p) {
 }
 
 // From 352 stripes on: below, the stream pass costs less (16 x 32 x 8 rows of
-// 88064: 250 us here, 246 there; of 95232: 247 and 259), as a row here costs
+// 88000: 247 us here, 240 there; of 95232: 247 and 259), as a row here costs
 // what its 32 chunks hold whatever its length.
 bool row_relay_preferred(const DecodeParams& p) { return (p.V + 255) / 256 >= 352; }
 

@@ -1528,10 +1528,11 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, 
 //     rows (the candidate set only grows, so rows that passed still pass);
 //   * the trace and the next state.
 // With constraints (CON: n-gram blocking of n >= 2, a repetition penalty)
-// each beam's prefix lives in LDS with a 32 W-bit signature (two hashed bits
-// per token), both double-buffered and rebuilt from the parent's at every
-// step; each step lists a read beam's n-gram-blocked tokens (one lane per
-// prefix position), and every candidate takes make_cand's value (blocked:
+// each beam's prefix lives in LDS with two 32 W-bit signatures (two hashed bits
+// per token, and per (n - 1)-gram), all double-buffered and copied from the
+// parent's at every step (Prefixes); a step lists a beam's n-gram-blocked
+// tokens (one lane per prefix position) where its last (n - 1)-gram may have
+// occurred before, and every candidate takes make_cand's value (blocked:
 // none; in the prefix: lp - log(rep)). Constraints only lower a value, so the
 // row pass's bound still covers every token left out, and tau counts on K of
 // a row's first K + nblk entries (a blocked token is one entry at most),
@@ -1747,7 +1748,10 @@ struct Prefixes {
 // CON: an entry whose token the beam's signature may hold is looked up in the
 // prefix by the whole wavefront, a beam whose last (n - 1)-gram may have
 // occurred lists its blocked tokens, and a row's entries from J on are left
-// out like those of the list's end: the last one held bounds them.
+// out like those of the list's end: the last one held bounds them. 3.0 us a
+// step at 128 steps (the general step, its prefixes rebuilt with per-lane
+// addresses and searched by one lane a candidate: 6.0): 64 x 128 x 5 x 50257
+// f16, n-gram 3 and a penalty, 860 -> 433 us.
 // Returns the first step not taken: steps_b, or a step whose rows need a
 // full read or whose words never came (gave_up). s: 64 keys of 16 bytes, then
 // the selection (kGridBeams of 16 bytes, over the shortlists).

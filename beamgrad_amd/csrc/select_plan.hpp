@@ -29,7 +29,7 @@ constexpr int kWideRank = 4;  // candidates per thread of the rank compaction be
 
 // The narrow select pass (select_kernels.hpp).
 constexpr int kNarrowMaxK = 16;       // the running list lives in one 16-lane DPP row
-constexpr int kGridBeams = 8;         // beams whose K * K candidates fit one wavefront's lanes (grid_steps)
+constexpr int kGridBeams = 8;         // beams whose candidates fit one wavefront's lanes, K of each at least (grid_steps)
 constexpr int kGridAhead = 4;         // steps its words are loaded ahead
 constexpr int kGridAheadCon = 2;      // with constraints (longer steps, and twice the step's code instead of four times)
 constexpr int kNarrowPf = 4;          // 16-byte prefetch registers per lane (K * M <= 512)
