@@ -1729,11 +1729,13 @@ struct Prefixes {
 
 // The steps of a decode of at most kGridBeams beams, the candidates in a
 // grid: lane (k, j) = k J + j holds entry j of beam k's shortlist (J = K
-// unconstrained, where only the first K of a list can be selected; as many
-// as 64 lanes hold with constraints) and every lane of beam k its state, so that a step moves nothing between lanes but the
+// unconstrained, where the entries from K on can be selected only on a tie
+// of raws, below; as many as 64 lanes hold with constraints) and every lane of
+// beam k its state, so that a step moves nothing between lanes but the
 // candidates' keys and the selection, through LDS:
 //   * the lane's entry and its row's RowInfo, loaded kGridAhead steps ahead
-//     (three words; a step's chain is shorter than a load's latency);
+//     (three words, and unconstrained the entry after the lane's; a step's
+//     chain is shorter than a load's latency);
 //   * tau, the largest K-th entry's raw: candidates below it are not selected;
 //   * the keys of the others, packed in LDS, and each one's rank among them:
 //     (raw, parent, token) where every beam is expanded (one length: the score
@@ -1765,10 +1767,11 @@ struct GridState {
 
 struct GridWords {
     uint32_t lp, tok;         // the entry (its tag in tok in the overlapped decode)
+    uint32_t nlp, ntok;       // the entry after it (unconstrained)
     uint32_t i0, i1, i2, i3;  // the row's RowInfo (tags in i1 and i3)
 };
 
-template <bool LOGITS, bool CON>
+template <int DT, bool LOGITS, bool CON>
 __device__ __forceinline__ int grid_steps(const DecodeParams& p, int b, int t, int steps_b, int Kb, int eos_b,
                                           GridState& g, Prefixes& pre, uint4* s_key, const float* s_pen,
                                           const float* s_inv, int pen_len, int lane, bool& any_invalid, int& first_bad,
@@ -1800,15 +1803,29 @@ __device__ __forceinline__ int grid_steps(const DecodeParams& p, int b, int t, i
         const int64_t row = ex + static_cast<int64_t>(tn < steps_b ? tn : steps_b - 1) * K + kc;
         const uint32_t* e = reinterpret_cast<const uint32_t*>(p.shortlist + row * M + jc);
         const uint32_t* r = reinterpret_cast<const uint32_t*>(p.rowinfo + row);
+        // (the entry after the last of a list is the next row's, or past the
+        // last row's a word of the workspace's counters: read, not used)
         if (coherent) {
             (void)read_tagged(e, w.lp, w.tok);
+            if constexpr (!CON) (void)read_tagged(e + 2, w.nlp, w.ntok);
             (void)read_tagged(r, w.i0, w.i1);
             (void)read_tagged(r + 2, w.i2, w.i3);
         } else {
-            const uint2 ev = *reinterpret_cast<const uint2*>(e);
+            // (both entries in one load, 8-byte aligned: a load of its own for
+            // the second one cost 0.2 us a step)
+            struct __attribute__((packed, aligned(8))) Entries { uint32_t lp, tok, nlp, ntok; };
+            if constexpr (CON) {
+                const uint2 ev = *reinterpret_cast<const uint2*>(e);
+                w.lp = ev.x;
+                w.tok = ev.y;
+            } else {
+                const Entries ev = *reinterpret_cast<const Entries*>(e);
+                w.lp = ev.lp;
+                w.tok = ev.tok;
+                w.nlp = ev.nlp;
+                w.ntok = ev.ntok;
+            }
             const uint4 iv = *reinterpret_cast<const uint4*>(r);
-            w.lp = ev.x;
-            w.tok = ev.y;
             w.i0 = iv.x;
             w.i1 = iv.y;
             w.i2 = iv.z;
@@ -1821,11 +1838,15 @@ __device__ __forceinline__ int grid_steps(const DecodeParams& p, int b, int t, i
         const bool carried = live && eos_b >= 0 && g.ended != 0;
         const bool read = live && !carried;
         uint32_t lpw = w.lp, tokw = w.tok, i0 = w.i0, i1 = w.i1, i2 = w.i2, i3 = w.i3;
+        uint32_t nlpw = CON ? 0u : w.nlp;
+        const bool last_held = !CON && j == J - 1;  // (its next entry is the row's first not held)
+        const uint32_t w_ntok = CON ? 1u : w.ntok;
         issue(w, tt + AHEAD);
         if (coherent) {
             // words not yet written (tag 0) are waited for
             const bool miss_info = read && (i1 == 0u || i3 == 0u);
-            if (__builtin_amdgcn_ballot_w64(miss_info || (read && tokw == 0u)) != 0) {
+            const bool miss_next = !CON && last_held && w_ntok == 0u;
+            if (__builtin_amdgcn_ballot_w64(miss_info || (read && (tokw == 0u || miss_next))) != 0) {
                 const int64_t row = ex + static_cast<int64_t>(tt) * K + kc;
                 const uint32_t* e = reinterpret_cast<const uint32_t*>(p.shortlist + row * M + jc);
                 const uint32_t* r = reinterpret_cast<const uint32_t*>(p.rowinfo + row);
@@ -1834,6 +1855,8 @@ __device__ __forceinline__ int grid_steps(const DecodeParams& p, int b, int t, i
                     if (i1 == 0u) ok = wait_tagged(p, r, i0, i1);
                     if (ok && i3 == 0u) ok = wait_tagged(p, r + 2, i2, i3);
                     if (ok && tokw == 0u && jc < static_cast<int>(i1) - 2) ok = wait_tagged(p, e, lpw, tokw);
+                    uint32_t tag = 1u;
+                    if (ok && miss_next && J < static_cast<int>(i1) - 2) ok = wait_tagged(p, e + 2, nlpw, tag);
                 }
                 if (__builtin_amdgcn_ballot_w64(!ok) != 0) {
                     gave_up = true;
@@ -1854,6 +1877,27 @@ __device__ __forceinline__ int grid_steps(const DecodeParams& p, int b, int t, i
         int token = static_cast<int>(tokw);
         bool have = read && j < cnt;
         uint32_t tail = 0u;
+        // What bounds the entries past those held. (Unconstrained, the first
+        // of them: K others of the row have no lower raw, but log-probs that
+        // differ can give one raw, and then the lower token comes first.)
+        float left = bound;
+        if constexpr (CON) {
+            left = j == J - 1 && cnt > J && lp > bound ? lp : bound;
+        } else {
+            bool first_out = j == J - 1 && cnt > J;
+            if constexpr (DT != 0) {
+                // 16-bit rows often have one value on both sides of K, which
+                // would fail the check below. Where the neighbours of that
+                // value (2^-9 of a bfloat16 away at least, 2^-12 of a binary16)
+                // are further off than the additions round (2^-22 of the
+                // sums), the entries of one raw are in the order of their
+                // tokens, and K of the row do come first.
+                const float value = LOGITS ? lp + lse : lp;
+                const float sums = __builtin_fabsf(g.raw) + __builtin_fabsf(lp) + __builtin_fabsf(lse);
+                first_out = first_out && !(nlpw == lpw && __builtin_fabsf(value) * (DT == 1 ? 0x1p-12f : 0x1p-9f) > sums * 0x1p-20f);
+            }
+            if (first_out) left = bits_f32(nlpw);
+        }
         if constexpr (CON) {
             // (a read beam's prefix holds tt tokens)
             const int n = p.ngram;
@@ -1949,19 +1993,13 @@ __device__ __forceinline__ int grid_steps(const DecodeParams& p, int b, int t, i
         wave_sync();
         const uint4 mine = s_sel[kc];
         const uint4 kth = s_sel[Kb - 1];
-        // Exactness: every candidate left out of a row's list (unconstrained,
-        // its entries from K on too: K others of the row come first; else
-        // those past the last one held) has raw <= fl(p + bound); the row
-        // passes when the Kb-th selected candidate ranks strictly before that
-        // bound's score and raw.
-        bool fail = read && cnt < 0;
-        const float left = CON && j == J - 1 && cnt > J && lp > bound ? lp : bound;
-        if (read && left > -kInf) {
-            const float X = g.raw + left;
-            const float SX = X * inv;
-            const float ks = nsel >= Kb ? bits_f32(kth.x) : -kInf, kr = nsel >= Kb ? bits_f32(kth.y) : -kInf;
-            fail = fail || (X > -kInf && !((ks > SX) || (ks == SX && kr > X)));
-        }
+        // Exactness: every candidate left out of a row's list, those past the
+        // last entry held too, has raw <= fl(p + left); the row passes when the
+        // Kb-th selected candidate ranks strictly before that score and raw.
+        const float ks = nsel >= Kb ? bits_f32(kth.x) : -kInf, kr = nsel >= Kb ? bits_f32(kth.y) : -kInf;
+        const float X = g.raw + left;
+        const float SX = X * inv;
+        const bool fail = read && (cnt < 0 || (X > -kInf && !((ks > SX) || (ks == SX && kr > X))));
         if (__builtin_amdgcn_ballot_w64(fail) != 0) return false;
         if (bad_m != 0) {
             any_invalid = true;
@@ -2148,8 +2186,8 @@ __device__ __forceinline__ void narrow_example(const DecodeParams& p, int pen_le
     for (int t = 0; t < T; ++t) {
         if (grid && t < steps_b && !gave_up) {
             GridState g{__shfl(raw, gk), __shfl(len, gk), __shfl(last, gk), __shfl(ended ? 1 : 0, gk)};
-            t = grid_steps<LOGITS, CON>(p, b, t, steps_b, Kb, eos_b, g, pre, s_key, s_pen, s_inv, pen_len, lane,
-                                        any_invalid, first_bad, gave_up);
+            t = grid_steps<DT, LOGITS, CON>(p, b, t, steps_b, Kb, eos_b, g, pre, s_key, s_pen, s_inv, pen_len, lane,
+                                            any_invalid, first_bad, gave_up);
             const int src = lane < K ? lane * gJ : 0;
             const float raw_k = __shfl(g.raw, src);  // (every lane shuffles)
             const int ended_k = __shfl(g.ended, src);
