@@ -2126,7 +2126,7 @@ __device__ __forceinline__ void narrow_example(const DecodeParams& p, int pen_le
     // below, and only those that fail its exactness check (and the padding
     // steps) through the general step. (The test knob for waits that give up
     // forces the general step's counted wait.)
-    const bool grid = K <= kGridBeams && M >= K && p.wait_extra == 0;
+    const bool grid = grid_fits(K, M, T) && p.wait_extra == 0;
     if constexpr (PF) {
         have_pf = steps_b > 0 && !grid;
         if (have_pf) prefetch(0);

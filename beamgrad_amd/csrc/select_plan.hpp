@@ -40,6 +40,15 @@ constexpr int kNarrowWaves = 4;       // examples (wavefronts) per workgroup, at
 constexpr int kXcds = 8;              // MI355X: 8 XCDs of 32 CUs
 constexpr int kNarrowWaveLds = 24576; // LDS per wavefront, at most (else the workgroup pass)
 
+// Whether a decode's steps go through the grid of candidates: lists at least
+// as long as the beams, and a trace whose byte offsets (an example's, past the
+// end included) fit in 31 bits.
+constexpr bool grid_fits(int K, int M, int T) {
+    return K <= kGridBeams && M >= K && static_cast<int64_t>(T) * K < (1 << 29);
+}
+static_assert(grid_fits(8, 24, 1 << 25) && !grid_fits(9, 24, 1) && !grid_fits(4, 3, 1), "beams and lists");
+static_assert(!grid_fits(8, 24, 1 << 26) && !grid_fits(1, 24, 1 << 29) && grid_fits(1, 24, (1 << 29) - 1), "offsets");
+
 // The prefetch needs the row pass finished before the select pass starts (not
 // the overlapped decode, whose rows land while it runs) and a step's
 // shortlists within the prefetch registers, as 16-byte pairs of entries.
