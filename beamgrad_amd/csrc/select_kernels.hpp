@@ -1293,8 +1293,9 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, 
         if constexpr (WIDE) {
             // Constrained, stepped, or too many at once: entry i of every list
             // in turn, best first, until no list's entry could be admitted
-            // (a list is sorted, so neither could its later ones; penalties
-            // only lower a candidate).
+            // whatever its token (a list is sorted by log-prob, so neither
+            // could its later ones, of which one of the same raw may have a
+            // lower token; penalties only lower a candidate).
             if (M > 0 && !one_pass && forced < 0) {
                 const float tau = st.tau;
                 for (int i = 0; i < M; ++i) {
@@ -1309,7 +1310,7 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, 
                             const int new_len = s.len[k] + 1;
                             const float inv = inv_of(s, pen_len, new_len, p.alpha);
                             const float raw0 = praw + e.lp;
-                            if (!(raw0 < tau) && !before(st.thr, Cand{raw0 * inv, raw0, k, e.token, new_len, 1})) {
+                            if (!(raw0 < tau) && !before(st.thr, Cand{raw0 * inv, raw0, k, -1, new_len, 1})) {
                                 st.overflow = 1;
                                 const PrefixView pre = prefix_of(p, s, b, k, cur);
                                 Cand c;

@@ -92,3 +92,55 @@ def test_equal_log_probs(hip, oracle, K, dtype):
     x[:, 0] -= 4000.0
     x[4:, 1:] *= np.float32(2.0 ** -13)  # far below the raw's ulp
     _check(hip, oracle, x, dtype, -1, eos_token=-1, alpha=0.6)
+
+
+def _wide_rows():
+    """72 beams: after a first step near -30000, 71 rows give one good entry
+    each, and 80 entries of the last row share the raw of the 72nd place. Its
+    lowest token stands past one that ranks after the eleven before it."""
+    B, T, K, V, R = 2, 3, 72, 700, -30005.0
+    rng = np.random.default_rng(5)
+    x = rng.uniform(-20000.0, -19000.0, size=(B, T, K, V)).astype(np.float32)
+    first = (-30000.0 + np.arange(K)[::-1] * 2.0 ** -7).astype(np.float32)
+    x[:, 0, 0] -= 30000.0
+    x[:, 0, 0, 100:100 + K] = first
+    for k in range(K - 1):
+        x[:, 1, k, 650] = np.float32(R + 1.0) - first[k]
+    tokens = np.concatenate([np.arange(600, 611), [680], np.arange(300, 368)[::-1]])
+    lp = (np.float64(R) - np.float64(first[K - 1]) + 4e-4 - 1e-5 * np.arange(80)).astype(np.float32)
+    assert len(np.unique(lp)) == 80 and np.all(first[K - 1] + lp == np.float32(R))
+    x[:, 1, K - 1, tokens] = lp
+    return x
+
+
+@pytest.mark.parametrize("overlap", [0, 1])
+def test_wide_lists_in_rounds(hip, oracle, overlap):
+    _check(hip, oracle, _wide_rows(), "f32", overlap, eos_token=-1, alpha=0.6, repetition_penalty=1.2)
+
+
+def test_wide_lists_step_api(hip, oracle):
+    x = _wide_rows()
+    want = oracle.decode(x, dtype="f32", eos_token=-1, alpha=0.6)
+    got = hip.steps(x, "f32", eos_token=-1, alpha=0.6)
+    for name in got:
+        a, b = np.asarray(got[name]), np.asarray(want[name])
+        assert np.array_equal(a.view(np.uint32) if a.dtype == np.float32 else a,
+                              b.view(np.uint32) if b.dtype == np.float32 else b), name
+
+
+@pytest.mark.parametrize("K", [12, 24, 64, 65, 130, 300])
+@pytest.mark.parametrize("constrained", [False, True])
+def test_more_beams(hip, oracle, K, constrained):
+    """Past the grid, where every entry that reaches tau is a candidate."""
+    rng = np.random.default_rng(K)
+    x = rng.uniform(-90.0, -50.0, size=(2, 4, K, 900)).astype(np.float32)
+    x[:, 0] -= 300.0
+    for b in range(2):
+        for t in range(4):
+            for k in range(K):
+                n = int(rng.integers(1, 100))
+                tokens = np.sort(rng.choice(900, size=n, replace=False))[::-1]
+                top = (-300.0 if t == 0 else -1.5) - 0.25 * float(rng.integers(0, 3))
+                x[b, t, k, tokens] = _ladder(top, n)
+    kw = dict(no_repeat_ngram_size=2, repetition_penalty=1.3) if constrained else {}
+    _check(hip, oracle, x, "f32", -1, eos_token=-1, alpha=0.6, **kw)
