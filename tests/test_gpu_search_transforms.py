@@ -31,3 +31,46 @@ def test_dual_rows_are_refused(enabled, dual_step):
         # rows without a tangent inside a level are plain rows
         scores = bg.beam_search(lambda s: rows[s.step], OPTS, 3, batch_size=2, device="cuda").scores
         assert forward_ad.unpack_dual(scores).tangent is None
+
+
+@pytest.mark.parametrize("max_steps", [1, 3])
+def test_last_step_is_not_waited_for(max_steps):
+    """Without validation, nothing follows from the last step's outcome."""
+    rows = _rows()
+    options = bg.BeamOptions(beam_size=3, eos_token=2, length_penalty_alpha=0.6, validate_inputs=False)
+    busy = torch.randn(8192, 8192, device="cuda")
+    queued = torch.cuda.Event()
+
+    def step(state):
+        if state.step + 1 == max_steps:
+            for _ in range(20):
+                busy @ busy  # tens of milliseconds ahead of the last step
+            queued.record()
+        return rows[state.step]
+
+    bg.beam_search(lambda s: rows[s.step], options, max_steps, batch_size=2, device="cuda")
+    busy @ busy
+    torch.cuda.synchronize()
+    bg.beam_search(step, options, max_steps, batch_size=2, device="cuda")
+    assert not queued.query()
+
+
+def test_outer_rows_under_transforms():
+    """The caller's own rows inside torch.func transforms, whose beams are wrapped."""
+    rows = _rows()
+
+    def weighted(w):
+        return (bg.beam_search(lambda s: rows[s.step], OPTS, 3, batch_size=2, device="cuda").scores * w).sum()
+
+    def first_step(x):
+        return bg.beam_search(lambda s: x if s.step == 0 else rows[s.step], OPTS, 3, batch_size=2,
+                              device="cuda").scores.sum()
+
+    scores = bg.beam_search(lambda s: rows[s.step], OPTS, 3, batch_size=2, device="cuda").scores
+    w = torch.arange(6.0, device="cuda").reshape(2, 3)
+    assert torch.equal(torch.func.grad(weighted)(w), scores)
+    value, tangent = torch.func.jvp(weighted, (w,), (w,))
+    assert torch.equal(value, (scores * w).sum()) and torch.equal(tangent, value)
+    x = rows[0].clone().requires_grad_(True)
+    first_step(x).backward()
+    assert torch.equal(torch.func.grad(first_step)(rows[0]), x.grad)
