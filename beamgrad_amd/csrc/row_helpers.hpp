@@ -123,6 +123,30 @@ __device__ __forceinline__ uint32_t term_slots(uint32_t R) {
     return idx | ((R >> 3) & 0x10001000u);
 }
 
+// The lowest finite value of an input type: a threshold at it lists every
+// finite entry.
+template <int DT>
+__device__ __forceinline__ float lowest_finite() {
+    return DT == 0 ? -3.4028234663852886e38f : (DT == 1 ? -65504.0f : -3.3895313892515355e38f);
+}
+
+// The shortlist threshold of a row without NaN / +inf, from the M-th largest of
+// its lane maxima (-inf, or NaN once its key is cut, where fewer than M lanes
+// hold a finite entry). A row with few finite entries (logits masked by a
+// grammar, or a top-k or top-p filter) lists them all, and nothing bounds what
+// is left out (list_bound); with each such row read in full by the select pass, a
+// decode of 16 x 64 x 4 x 50257 f32 logits of 10 finite entries took 17.5 ms,
+// with the lists 0.38.
+template <int DT>
+__device__ __forceinline__ float list_threshold(float mth) {
+    return mth >= lowest_finite<DT>() ? mth : lowest_finite<DT>();
+}
+// The bound on the entries left out of a list of at most M survivors.
+template <int DT>
+__device__ __forceinline__ float list_bound(float theta) {
+    return theta > lowest_finite<DT>() ? theta : -kInf;
+}
+
 // Inverse of key16.
 __device__ __forceinline__ uint32_t key_pattern(int key) {
     return static_cast<uint16_t>(key < 0 ? (key ^ 0x7fff) : key);

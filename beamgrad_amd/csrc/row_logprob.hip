@@ -273,8 +273,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(C <= 32 && N
         }
         __syncthreads();
         if (tid == kTicketThread) s_bad = 0;  // every thread has read it
-        const float theta = (M > 0 && !any_bad) ? s_theta : -kInf;
-        const bool full = M > 0 && !(theta > -kInf);  // no shortlist: every element would survive
+        const bool full = M > 0 && any_bad;  // no shortlist
+        const float theta = (M > 0 && !any_bad) ? list_threshold<DT>(s_theta) : -kInf;
 
         // Blocks that can hold survivors (maximum >= theta) are copied to LDS.
         if (M > 0 && !full && tmax >= theta) {
@@ -379,7 +379,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(C <= 32 && N
             if (M > 0) {
                 if (listed) {
                     info.count = n < M ? n : M;
-                    info.bound = n > M ? s_bound : theta;
+                    info.bound = n > M ? s_bound : list_bound<DT>(theta);
                 } else {
                     info.count = -1;
                 }

@@ -94,10 +94,9 @@ __global__ __launch_bounds__(kShortThreads) __attribute__((amdgpu_waves_per_eu(C
     for (int e = 0; e < 4; ++e) k4[e] = ordered_key(top[e]);
     const float m = wave_max_dpp(key_value(max(max(k4[0], k4[1]), max(k4[2], k4[3]))));
     const bool do_lse = m > -kInf;
+    const bool listing = M > 0 && !any_bad;  // (a flagged row keeps no shortlist)
     float theta = -kInf;
-    if (M > 0 && !any_bad) theta = key_value(mth_largest_key<32, 12>(k4, M));
-    // no shortlist: a flagged row, or one whose every entry would survive
-    const bool listing = M > 0 && !any_bad && theta > -kInf;
+    if (listing) theta = list_threshold<DT>(key_value(mth_largest_key<32, 12>(k4, M)));
 
     float lse = 0.0f;
     if constexpr (LOGITS) {
@@ -156,7 +155,7 @@ __global__ __launch_bounds__(kShortThreads) __attribute__((amdgpu_waves_per_eu(C
     }
     if (M > 0 && (!listing || n > kShortSurvivors)) n = kSurvivorCap + 1;  // (no shortlist)
     wave_sync();
-    finish_row_wave<LOGITS>(p, r, lse, theta, any_bad, s_key, s_x, n, lane);
+    finish_row_wave<LOGITS>(p, r, lse, list_bound<DT>(theta), any_bad, s_key, s_x, n, lane);
 }
 
 template <int DT, bool LOGITS, int C>

@@ -182,9 +182,8 @@ row_stream_kernel(DecodeParams p, int64_t rows) {
         if (tid == kTicketThread) s_bad = 0;  // every thread has read it
         const float m = s_m;
         const bool do_lse = m > -kInf;  // (log-probs: a finite entry)
-        // no shortlist: a flagged row, or one whose every element would survive
-        const bool listing = M > 0 && !any_bad && s_theta > -kInf;
-        const float theta = listing ? s_theta : kInf;
+        const bool listing = M > 0 && !any_bad;  // (a flagged row keeps no shortlist)
+        const float theta = listing ? list_threshold<DT>(s_theta) : kInf;
 
         bool table = false;
         if constexpr (TABLE) {
@@ -355,7 +354,7 @@ row_stream_kernel(DecodeParams p, int64_t rows) {
             if (M > 0 && (do_lse || !LOGITS)) {
                 if (listed) {
                     info.count = n < M ? n : M;
-                    info.bound = n > M ? s_bound : theta;
+                    info.bound = n > M ? s_bound : list_bound<DT>(theta);
                     if constexpr (LOGITS) info.bound = info.bound - lse;
                 } else {
                     info.count = -1;
