@@ -729,10 +729,13 @@ bool row_relay_eligible(const DecodeParams& p) {
     return p.M <= 256;
 }
 
-// From 352 stripes on: below, the stream pass costs less (16 x 32 x 8 rows of
-// 88000: 247 us here, 240 there; of 95232: 247 and 259), as a row here costs
-// what its 32 chunks hold whatever its length.
-bool row_relay_preferred(const DecodeParams& p) { return (p.V + 255) / 256 >= 352; }
+// From 456 stripes (116481 entries) on. A row here costs what its 32 chunks hold
+// whatever its length, and rows with a maximum below 1 keep no shortlist (the
+// select pass reads them in full: logits with their maximum subtracted, 16 x 32
+// x 8 x 100352, take 67 ms; log-probs passed as logits likewise), so the rows
+// where the stream pass is about as fast go there: the row pass of 16 x 32 x 8
+// rows of 95232 takes 247 us here and 259 there, of 88000 247 and 240.
+bool row_relay_preferred(const DecodeParams& p) { return (p.V + 255) / 256 >= (3 * kRlStripes) / 4; }
 
 hipError_t launch_row_relay(const DecodeParams& p, int64_t rows, hipStream_t stream) {
     int device = 0;

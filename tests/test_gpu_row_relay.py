@@ -178,3 +178,27 @@ def test_stream_overlapped_select(stream, oracle, overlap):
     finally:
         lib.dbs_hip_profile_enable(0)
         lib.dbs_hip_set_decode_overlap(prev)
+
+
+@pytest.mark.parametrize("V", [89864, 100352, 102400, 116480])
+def test_shorter_rows_below_one_keep_their_lists(hip, oracle, V):
+    """bfloat16 logits with their maximum subtracted (no row reaches 1, where
+    this pass keeps no list) of lengths this pass does not take: no row is read
+    in full by the select pass."""
+    import ctypes as C
+
+    rng = np.random.default_rng(V)
+    x = rng.normal(0.0, 3.0, size=(2, 3, 4, V)).astype(np.float32)
+    x -= x.max(-1, keepdims=True)
+    xin = to_bits(x, "bf16")
+    kw = dict(from_logits=True, eos_token=5, alpha=0.6)
+    want = oracle.decode(xin, dtype="bf16", **kw)
+    hip.lib.dbs_hip_profile_enable(1)
+    try:
+        got = hip.decode(xin, "bf16", **kw)
+        ms, n = C.c_double(), C.c_int64()
+        assert hip.lib.dbs_hip_profile_read(5, C.byref(ms), C.byref(n)) == 0
+    finally:
+        hip.lib.dbs_hip_profile_enable(0)
+    assert first_difference(got, want) is None, first_difference(got, want)
+    assert n.value == 0
