@@ -264,6 +264,21 @@ DecodeLayout fitting_layout(const void* workspace, int64_t workspace_bytes, int 
     return workspace_bytes >= static_cast<int64_t>(small.total) ? small : L;
 }
 
+// Scratch for layout L, which without a caller's workspace becomes the one
+// without shortlists beyond 64 beams where the device has no room for them.
+hipError_t acquire_layout(Scratch& scratch, DecodeLayout& L, void* workspace, int64_t workspace_bytes,
+                          const DBSCudaDecodeArgs& a, bool step_mode, int prefix_stride, int keep, hipStream_t stream,
+                          bool* too_small) {
+    hipError_t e = scratch.acquire(workspace, workspace_bytes, L.total, stream, too_small);
+    if (e == hipSuccess || workspace) return e;
+    const DecodeLayout small = decode_layout(a.batch_size, step_mode ? 1 : a.steps, a.beam_size, a.vocab_size,
+                                             constrained(a), step_mode, prefix_stride, keep, false);
+    if (small.total >= L.total) return e;
+    (void)hipGetLastError();
+    L = small;
+    return scratch.acquire(workspace, workspace_bytes, L.total, stream, too_small);
+}
+
 int decode_common(const void* inputs, int data_type, int from_logits, const DBSCudaDecodeArgs* args,
                   const DBSCudaSearchOptions* options, const uint8_t* banned_pe, const DBSCudaDecodeOutputs* outputs,
                   float* row_lse, void* workspace, int64_t workspace_bytes, void* stream_ptr,
@@ -278,11 +293,12 @@ int decode_common(const void* inputs, int data_type, int from_logits, const DBSC
     const int pool_mult = pool ? pool->mult : 0;
     if (pool_mult < 0 || static_cast<int64_t>(pool_mult) * a.beam_size > DBS_CUDA_MAX_BEAM)
         return DBS_CUDA_STATUS_INVALID_ARGUMENT;
-    const DecodeLayout L = fitting_layout(workspace, workspace_bytes, a.batch_size, a.steps, a.beam_size, a.vocab_size,
-                                          cons, false, 0, pool_mult * a.beam_size);
+    DecodeLayout L = fitting_layout(workspace, workspace_bytes, a.batch_size, a.steps, a.beam_size, a.vocab_size, cons,
+                                    false, 0, pool_mult * a.beam_size);
     bool too_small = false;
     Scratch scratch;
-    hipError_t e = scratch.acquire(workspace, workspace_bytes, L.total, stream, &too_small);
+    hipError_t e = acquire_layout(scratch, L, workspace, workspace_bytes, a, false, 0, pool_mult * a.beam_size, stream,
+                                  &too_small);
     if (too_small) return DBS_CUDA_STATUS_INVALID_ARGUMENT;
     if (e != hipSuccess) return finish(stream, e);
     char* ws = static_cast<char*>(scratch.ptr);
@@ -358,12 +374,13 @@ int step_common(const void* inputs, int data_type, int from_logits, const DBSCud
         return DBS_CUDA_STATUS_INVALID_ARGUMENT;
     DecodeLayout L = fitting_layout(workspace, workspace_bytes, a.batch_size, 1, a.beam_size, a.vocab_size, cons, true,
                                     state->prefix_stride, pool_mult * a.beam_size);
-    if (row_mask) L.M = 0;  // filtered rows are read in full
     bool too_small = false;
     Scratch scratch;
-    hipError_t e = scratch.acquire(workspace, workspace_bytes, L.total, stream, &too_small);
+    hipError_t e = acquire_layout(scratch, L, workspace, workspace_bytes, a, true, state->prefix_stride,
+                                  pool_mult * a.beam_size, stream, &too_small);
     if (too_small) return DBS_CUDA_STATUS_INVALID_ARGUMENT;
     if (e != hipSuccess) return finish(stream, e);
+    if (row_mask) L.M = 0;  // filtered rows are read in full
     char* ws = static_cast<char*>(scratch.ptr);
     const int checked = check_per_example(a, reinterpret_cast<int32_t*>(ws + L.off_rowinfo), stream);
     if (checked != DBS_CUDA_STATUS_OK) return checked;
@@ -500,13 +517,14 @@ int step_for_host(const void* inputs, int data_type, int from_logits, const DBSC
                        workspace_bytes, stream, forced, pool, row_mask);
 }
 
-int64_t workspace_for_host(const DBSCudaDecodeArgs* args, int pool_mult, int step_mode, int prefix_stride) {
+int64_t workspace_for_host(const DBSCudaDecodeArgs* args, int pool_mult, int step_mode, int prefix_stride,
+                           bool wide_lists) {
     if (!valid_args(args) || pool_mult < 0 || static_cast<int64_t>(pool_mult) * args->beam_size > DBS_CUDA_MAX_BEAM)
         return -1;
     if (step_mode && (args->steps != 1 || args->steps_per_example || prefix_stride < 0)) return -1;
     return static_cast<int64_t>(decode_layout(args->batch_size, step_mode ? 1 : args->steps, args->beam_size,
                                               args->vocab_size, constrained(*args), step_mode != 0,
-                                              step_mode ? prefix_stride : 0, pool_mult * args->beam_size)
+                                              step_mode ? prefix_stride : 0, pool_mult * args->beam_size, wide_lists)
                                     .total);
 }
 
@@ -856,6 +874,10 @@ DBS_CUDA_EXPORT int dbs_hip_backtrack(const int32_t* tokens, const int32_t* pare
     hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
     return finish(stream,
                   launch_backtrack(tokens, parents, steps_per_example, batch_size, steps, beam_size, sequences, stream));
+}
+
+int64_t beamgrad_least_workspace(const DBSCudaDecodeArgs* args, int step_mode, int prefix_stride) {
+    return workspace_for_host(args, 0, step_mode, prefix_stride, false);
 }
 
 int beamgrad_advance_beams(const int32_t* tokens, const int32_t* parents, const int32_t* lengths,

@@ -236,9 +236,15 @@ void run_decode(DBSDecoderHandle* h, const DecodeJob& j) {
     int32_t* first_invalid =
         h->validate ? static_cast<int32_t*>(h->arena.get(kFirstInvalid, sizeof(int32_t) * static_cast<size_t>(B)))
                     : nullptr;
-    const int64_t ws_bytes = dbs_hip::workspace_for_host(&a, pool.mult, 0, 0);
+    int64_t ws_bytes = dbs_hip::workspace_for_host(&a, pool.mult, 0, 0);
     need(ws_bytes > 0, "invalid decode arguments");
-    void* ws = h->arena.get(kWorkspace, static_cast<size_t>(ws_bytes));
+    void* ws = nullptr;
+    try {
+        ws = h->arena.get(kWorkspace, static_cast<size_t>(ws_bytes));
+    } catch (const std::bad_alloc&) {
+        ws_bytes = dbs_hip::workspace_for_host(&a, pool.mult, 0, 0, false);
+        ws = h->arena.get(kWorkspace, static_cast<size_t>(ws_bytes));
+    }
     int32_t* fault = nullptr;
     engine_check(dbs_hip::decode_for_host(x, j.data_type, j.from_logits ? 1 : 0, &a, &opts, banned_pe, &o, row_lse,
                                           first_invalid, forced, P > 0 ? &pool : nullptr, ws, ws_bytes, st, &fault),

@@ -42,8 +42,11 @@ struct PoolGrads {
 
 // Workspace bytes of decode_for_host (step_mode 0) or step_for_host
 // (step_mode 1, prefix_stride as dbs_cuda_decode_step_workspace_size) with a
-// relaxed pool of pool_mult (0: none); -1 for invalid arguments.
-int64_t workspace_for_host(const DBSCudaDecodeArgs* args, int pool_mult, int step_mode, int prefix_stride);
+// relaxed pool of pool_mult (0: none); -1 for invalid arguments. wide_lists
+// false: the least a decode takes, without the shortlists of more than 64
+// beams (its rows are then read in full).
+int64_t workspace_for_host(const DBSCudaDecodeArgs* args, int pool_mult, int step_mode, int prefix_stride,
+                           bool wide_lists = true);
 
 // dbs_hip_decode_ex3 (per-example banned masks [B, V] or null), plus
 // first_invalid (device int32 [B] or null): the first row holding NaN or

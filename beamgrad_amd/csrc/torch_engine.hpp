@@ -6,6 +6,14 @@
 
 #include <stdint.h>
 
+#include "dbs_cuda.h"
+
+// The least workspace a decode (step_mode 0) or a step takes: beyond 64 beams,
+// without the shortlists that dbs_cuda_decode_workspace_size and
+// dbs_cuda_decode_step_workspace_size make room for. -1 for invalid arguments.
+extern "C" __attribute__((visibility("default"))) int64_t beamgrad_least_workspace(const DBSCudaDecodeArgs* args,
+                                                                                   int step_mode, int prefix_stride);
+
 // The beams after one step of the step API, in one launch: from the step's
 // outputs and updated state [B, K] (tokens, parents, lengths, raw scores,
 // from_logprob, finished) and the sequences before it [B, K, step] (ignored at

@@ -117,3 +117,28 @@ def test_wide_without_room_for_lists(hip, oracle):
     rows = torch.randn(B, T, K, V, generator=torch.Generator().manual_seed(5)).log_softmax(-1).numpy()
     got = hip.decode(rows, "f32", noalloc=True)
     assert first_difference(got, hip.decode(rows, "f32")) is None
+
+
+def test_wide_lists_without_memory_for_them():
+    """Where the device has no room for the lists (656 bytes a row against 16),
+    a decode through torch goes without them, as one with a smaller workspace
+    does: the same results, every row read in full."""
+    import torch
+
+    import beamgrad_amd as bg
+
+    B, T, K, V = 16, 128, 128, 4
+    x = torch.randn(B, T, K, V, generator=torch.Generator().manual_seed(3)).log_softmax(-1).cuda()
+    options = bg.BeamOptions(beam_size=K, eos_token=-1, length_penalty_alpha=0.6)
+    want = [t.clone() for t in bg.decode(x, options)]
+    lists = 80 * 8 * B * T * K  # 168 MB
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.empty_cache()
+    room = torch.cuda.memory_reserved() + lists // 2
+    torch.cuda.set_per_process_memory_fraction(room / total)
+    try:
+        got = bg.decode(x, options)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    for a, b in zip(got, want, strict=True):
+        assert torch.equal(a, b)
