@@ -305,6 +305,15 @@ bool wait_give_up_knob() {
     return env && env[0] == '1';
 }
 
+// `stream` waits for everything queued on `other`: through `done`, or, where
+// that fails, with the host waiting for `other`.
+hipError_t join_streams(hipStream_t stream, hipStream_t other, hipEvent_t done) {
+    hipError_t e = hipEventRecord(done, other);
+    if (e == hipSuccess) e = hipStreamWaitEvent(stream, done, 0);
+    if (e != hipSuccess) (void)hipStreamSynchronize(other);
+    return e;
+}
+
 void wait_policy(DecodeParams& p) {
     p.wait_ticks = 200000000ull;
     p.wait_extra = 0;
@@ -422,13 +431,18 @@ hipError_t launch_decode(const DecodeParams& p0, const DecodeLayout& L, hipStrea
     // streams onto a few hardware queues, shared once there are more
     // streams), and no select-pass wait may depend on a launch submitted
     // after it.
+    // Once a launch is made on the second stream, the caller's stream waits
+    // for it whatever fails: it uses the caller's rows and workspace, which the
+    // caller may free in its own stream's order when this returns.
     p.select_hold = hold ? 1 : 0;
     if (persistent) {
         if (e == hipSuccess) e = launch_row_pass(p, stream);
         if (e == hipSuccess) e = hipStreamWaitEvent(aux->stream, aux->start, 0);
-        if (e == hipSuccess) e = launch_select(p, L.sel, aux->stream);
-        if (e == hipSuccess) e = hipEventRecord(aux->done, aux->stream);
-        if (e == hipSuccess) e = hipStreamWaitEvent(stream, aux->done, 0);
+        if (e == hipSuccess) {
+            e = launch_select(p, L.sel, aux->stream);
+            const hipError_t joined = join_streams(stream, aux->stream, aux->done);
+            if (e == hipSuccess) e = joined;
+        }
     } else {
         DecodeParams early = p;
         early.claimed = claimed;
@@ -436,9 +450,11 @@ hipError_t launch_decode(const DecodeParams& p0, const DecodeLayout& L, hipStrea
         early.early_ticks = 20000;  // 200 us of the 100 MHz counter
         if (e == hipSuccess) e = launch_select(early, L.sel, stream);
         if (e == hipSuccess) e = hipStreamWaitEvent(aux->stream, aux->start, 0);
-        if (e == hipSuccess) e = launch_row_pass(p, aux->stream);
-        if (e == hipSuccess) e = hipEventRecord(aux->done, aux->stream);
-        if (e == hipSuccess) e = hipStreamWaitEvent(stream, aux->done, 0);
+        if (e == hipSuccess) {
+            e = launch_row_pass(p, aux->stream);
+            const hipError_t joined = join_streams(stream, aux->stream, aux->done);
+            if (e == hipSuccess) e = joined;
+        }
         DecodeParams late = early;
         late.early = 0;
         if (e == hipSuccess) e = launch_select(late, L.sel, stream);
