@@ -1185,6 +1185,9 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, 
         // A shortlist is sorted (log-prob desc), so the entries reaching tau
         // are a prefix of it: one thread per beam measures its prefix, then
         // offers it.
+        // (A sum that overflows to -inf is no candidate: the dead sentinel ranks
+        // before it. offer() leaves it out, and so does a tau that is finite.)
+        constexpr float kLowestRaw = -3.4028234663852886e38f;
         bool one_pass = false;
         if constexpr (WIDE) {
             if (H > 0 && p.use_tau && forced < 0) {
@@ -1194,7 +1197,7 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, 
                 // wavefront, one entry a lane (a thread walking a list of 80
                 // took 40 us a step).
                 lds_barrier();  // the carried beams are in
-                const float tau = st.tau;
+                const float tau = fmaxf(st.tau, kLowestRaw);
                 const int base = st.count;
                 int32_t* const found = s.nlen;  // the beams whose head does not hold them all (free until the selection)
                 auto put = [&](int slot, int k, const ShortEntry& e) __attribute__((always_inline)) {
@@ -1249,7 +1252,7 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, 
             // prefixes at consecutive collector slots, and the four
             // wavefronts copy them, lane k for beam k)
             if (tid < 64) {
-                const float tau = st.tau;
+                const float tau = fmaxf(st.tau, kLowestRaw);
                 const int k = tid;
                 int n = 0;
                 if (k < K) {

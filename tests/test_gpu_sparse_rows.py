@@ -98,3 +98,18 @@ def test_rows_filled_with_the_lowest_value(hip, oracle):
             x[np.isinf(x)] = lowest
             for kind in (AUTO, STREAM, SHORT):
                 _rescans(hip, oracle, x, dtype, kind, from_logits=logits, alpha=0.6)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("K", [3, 12, 17, 64, 80, 257])
+def test_sums_that_overflow(hip, oracle, K, dtype):
+    """Fewer candidates than beams, some of them sums below the lowest value:
+    such a sum is no candidate."""
+    lowest = np.finfo(np.float32).min if dtype == "f32" else np.float32(-3.3895314e38)
+    rng = np.random.default_rng(K)
+    for V in (5, 23):
+        x = rng.normal(0.0, 1.0, size=(2, 5, K, V)).astype(np.float32)
+        x[rng.random(x.shape) < 0.7] = lowest
+        for logits in (False, True):
+            for overlap in (0, 1):
+                _rescans(hip, oracle, x, dtype, AUTO, overlap=overlap, from_logits=logits, alpha=0.6, steps=[5, 2])
