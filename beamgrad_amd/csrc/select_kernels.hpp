@@ -546,6 +546,12 @@ __device__ __forceinline__ void end_round(Lds& s, State& st, int K, int sort_cap
     if (__builtin_expect(st.count > sort_cap - kSelectThreads, 0)) compact(s, st, K);  // (rare: out of line)
 }
 
+// The next float above x (finite or -inf).
+__device__ __forceinline__ float next_above(float x) {
+    const uint32_t u = f32_bits(x);
+    return x == 0.0f ? bits_f32(1u) : bits_f32((u & 0x80000000u) ? u - 1u : u + 1u);
+}
+
 // Every candidate of row `row` (beam k) that does not rank after the
 // threshold: a sweep over the row gathers the tokens whose score could reach
 // it, then their candidates are offered to the collector. With no threshold
@@ -583,9 +589,9 @@ __device__ __forceinline__ void rescan_row(const DecodeParams& p, Lds& s, State&
         if (!make_cand(p, s, pre, k, praw, inv_pen, v, new_len, lp, c)) return false;
         return !(c.score < least) && !before(thr, c);
     };
-    // A batch's scores, penalties apart (they only lower a candidate); NaN,
-    // which passes no test, where there is no finite entry.
-    auto scan = [&](int v0, float (&score)[kRescanPerThread]) __attribute__((always_inline)) {
+    // A batch's raw scores times `scale`, penalties apart (they only lower a
+    // candidate); NaN, which passes no test, where there is no finite entry.
+    auto scan = [&](int v0, float scale, float (&value)[kRescanPerThread]) __attribute__((always_inline)) {
         float xs[kRescanPerThread];
 #pragma unroll
         for (int j = 0; j < kRescanPerThread; ++j) {  // every load made, from a clamped index
@@ -596,7 +602,7 @@ __device__ __forceinline__ void rescan_row(const DecodeParams& p, Lds& s, State&
         for (int j = 0; j < kRescanPerThread; ++j) {
             const float lp = LOGITS ? xs[j] - lse : xs[j];
             const bool in = v0 + j * kSelectThreads + tid < V && lp < kInf && lp > -kInf;
-            score[j] = in ? (praw + lp) * inv_pen : __builtin_nanf("");
+            value[j] = in ? (praw + lp) * scale : __builtin_nanf("");
         }
     };
     int32_t* const tokens = s.rbuf;
@@ -608,7 +614,7 @@ __device__ __forceinline__ void rescan_row(const DecodeParams& p, Lds& s, State&
 #pragma unroll 1
             for (int v0 = 0; v0 < V; v0 += kSelectThreads * kRescanPerThread) {
                 float score[kRescanPerThread];
-                scan(v0, score);
+                scan(v0, inv_pen, score);
                 if (plain) {
 #pragma unroll
                     for (int j = 0; j < kRescanPerThread; ++j) best[j & 3] = fmaxf(best[j & 3], score[j]);
@@ -636,14 +642,21 @@ __device__ __forceinline__ void rescan_row(const DecodeParams& p, Lds& s, State&
         }
         if (tid == 0) st.rcount = 0;
         lds_barrier();
-        const float floor_score = fmaxf(least, thr.score);
+        // Up to a threshold of this row's penalty the candidates go by raw (the
+        // score is a nondecreasing function of it), and the raw of the threshold
+        // itself passes only where a token of this row could rank before it:
+        // where very many entries have that raw (rows masked with the type's
+        // lowest value, rows of one value) all of them would pass by score.
+        const bool by_raw = !(least > thr.score) && thr.raw * inv_pen == thr.score;
+        const float scale = by_raw ? 1.0f : inv_pen;
+        const float lowest = by_raw ? (k <= thr.parent ? thr.raw : next_above(thr.raw)) : fmaxf(least, thr.score);
 #pragma unroll 1
         for (int v0 = 0; v0 < V; v0 += kSelectThreads * kRescanPerThread) {
-            float score[kRescanPerThread];
-            scan(v0, score);
+            float value[kRescanPerThread];
+            scan(v0, scale, value);
             uint32_t pass = 0;
 #pragma unroll
-            for (int j = 0; j < kRescanPerThread; ++j) pass |= (score[j] >= floor_score ? 1u : 0u) << j;
+            for (int j = 0; j < kRescanPerThread; ++j) pass |= (value[j] >= lowest ? 1u : 0u) << j;
             while (pass != 0) {
                 const int j = __ffs(static_cast<int>(pass)) - 1;
                 pass &= pass - 1;

@@ -113,3 +113,25 @@ def test_sums_that_overflow(hip, oracle, K, dtype):
         for logits in (False, True):
             for overlap in (0, 1):
                 _rescans(hip, oracle, x, dtype, AUTO, overlap=overlap, from_logits=logits, alpha=0.6, steps=[5, 2])
+
+
+@pytest.mark.parametrize("alpha", [0.0, 0.6])
+@pytest.mark.parametrize("K", [8, 20, 64, 70])
+def test_full_reads_at_the_threshold(hip, oracle, monkeypatch, K, alpha):
+    """Every row read in full, with very many entries of the threshold's score:
+    rows of one value, of a few, masked with the lowest value; thresholds from
+    rows before and after the row read, and from finished beams."""
+    monkeypatch.setenv("DBS_HIP_SHORTLIST", "0")
+    rng = np.random.default_rng(K)
+    V = 4001
+    for rows in ("constant", "coarse", "lowest"):
+        x = np.zeros((2, 4, K, V), np.float32)
+        if rows == "coarse":
+            x = np.round(rng.normal(0.0, 1.0, size=x.shape)).astype(np.float32)
+        if rows == "lowest":
+            x = _sparse(K, x.shape, 12)
+            x[np.isinf(x)] = np.finfo(np.float32).min
+        x[..., 9] += 3.0  # beams finish
+        for kw in (dict(eos_token=-1), dict(eos_token=9, min_length=2), dict(eos_token=9, repetition_penalty=1.3)):
+            for logits in (False, True):
+                _rescans(hip, oracle, x, "f32", AUTO, from_logits=logits, alpha=alpha, **kw)
