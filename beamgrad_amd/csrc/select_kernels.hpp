@@ -543,7 +543,7 @@ __device__ __forceinline__ void offer(Lds& s, State& st, const Cand& c) {
 
 __device__ __forceinline__ void end_round(Lds& s, State& st, int K, int sort_cap) {
     lds_barrier();
-    if (__builtin_expect(st.count > sort_cap - kSelectThreads, 0)) compact(s, st, K);  // (rare: out of line)
+    if (st.count > sort_cap - kSelectThreads) compact(s, st, K);
 }
 
 // The next float above x (finite or -inf).
@@ -648,8 +648,9 @@ __device__ __forceinline__ void rescan_row(const DecodeParams& p, Lds& s, State&
         // where very many entries have that raw (rows masked with the type's
         // lowest value, rows of one value) all of them would pass by score.
         const bool by_raw = !(least > thr.score) && thr.raw * inv_pen == thr.score;
-        const float scale = by_raw ? 1.0f : inv_pen;
-        const float lowest = by_raw ? (k <= thr.parent ? thr.raw : next_above(thr.raw)) : fmaxf(least, thr.score);
+        auto uniform = [](float x) { return bits_f32(__builtin_amdgcn_readfirstlane(f32_bits(x))); };
+        const float scale = uniform(by_raw ? 1.0f : inv_pen);
+        const float lowest = uniform(by_raw ? (k <= thr.parent ? thr.raw : next_above(thr.raw)) : fmaxf(least, thr.score));
 #pragma unroll 1
         for (int v0 = 0; v0 < V; v0 += kSelectThreads * kRescanPerThread) {
             float value[kRescanPerThread];
@@ -702,7 +703,7 @@ __device__ __forceinline__ ShortEntry list_entry(const DecodeParams& p, State& s
 // paths keep their register budget.
 // HOLD: the kernel claims every accumulation register (a clobber of a255),
 // so no wavefront of another kernel fits on its SIMDs beside it: launched
-// before a row pass of one workgroup per row, it keeps its CUs to itself
+// before a row pass of several workgroups per CU, it keeps its CUs to itself
 // (registers it never uses; its own occupancy, one wavefront per SIMD, is
 // unchanged).
 // WIDE: more than kListBeams beams. The shortlists (shorter than the beams are
@@ -1389,7 +1390,7 @@ __global__ __launch_bounds__(kSelectThreads) void select_kernel(DecodeParams p, 
         // (Up to kListBeams beams rows rarely fail, and this is kept out of line:
         // in the steps' path, its loads' registers had the steps' own moved to and
         // from the accumulation registers. Select pass of 4 x 98 x 25 x 12106 f32
-        // log-probs 855 us, 777 so, of x 64 937 and 876. Beyond, where the first
+        // log-probs 855 us, 772 so, of x 64 937 and 877. Beyond, where the first
         // step's row always fails, out of line costs the rescan 5 %.)
         const int any_fail = __builtin_amdgcn_readfirstlane(st.any_fail);
         if (WIDE ? any_fail != 0 : __builtin_expect(any_fail, 0) != 0) {
