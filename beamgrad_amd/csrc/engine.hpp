@@ -39,7 +39,6 @@ constexpr int kRowThreads = 64;      // one wavefront per row in the row pass
 constexpr int kLanes = 256;          // lanes of the fixed logsumexp fold order
 constexpr int kSurvivorCap = 512;    // row-pass candidates kept per row before overflow
 constexpr int kSelectThreads = 256;  // one workgroup per example in the select pass
-constexpr int kRound = kSelectThreads;      // candidates offered per collector round (one per thread)
 
 // Per-row result of the row pass. In the overlapped decode every 8-byte
 // half of it, and every shortlist entry, is published as one 64-bit atomic
@@ -133,7 +132,7 @@ struct DecodeParams {
     int32_t* step_done;
     unsigned long long* row_ticket;
     int reserve_cus;  // CUs the persistent row-pass kernels leave free (the select pass's workgroups)
-    int select_hold;  // the select pass claims its SIMDs' registers (beside a row pass of one workgroup per row)
+    int select_hold;  // the select pass claims its SIMDs' registers (beside a row pass of several workgroups per CU)
     // A select-pass wait that gives up (bounded by wait_ticks of the 100 MHz
     // counter) sets *fault and marks its example invalid (2); the example's
     // remaining steps are written as padding. wait_extra raises the count a
