@@ -2,8 +2,8 @@
 """GPU parity of the surrogate backward through the C ABI
 (dbs_cuda_backward_ex, dbs_cuda_backward, dbs_hip_backward_dense,
 dbs_cuda_path_gradient), of the length penalty and of the backtrack, against
-the CPU oracle. Gradients are compared bit for bit (the north star allows 1e-6
-relative; the engine reproduces the reference's operation order)."""
+the CPU oracle. Gradients are compared bit for bit (the engine reproduces the reference's
+operation order)."""
 
 import numpy as np
 import pytest

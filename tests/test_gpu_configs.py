@@ -1,5 +1,5 @@
 # SPDX-License-Identifier: MIT
-"""The five BASELINE configurations at their full sizes on the GPU, checked
+"""The five headline configurations (C1 to C5) at their full sizes on the GPU, checked
 against the reference's own CPU library (oracle/_ref, where it is built; the
 oracle otherwise) on identical seeded inputs: every trace field and the final
 scores bit for bit, the logsumexp of every row (row_lse: the rows the search

@@ -3,9 +3,9 @@
 dbs_hip_decode_ex3) against the CPU oracle on identical seeded inputs.
 
 The bar is bit-exact for every field: tokens, parents, lengths, from_logprob,
-scores, raw scores, final scores, row logsumexp and the NaN/+inf flags. (The
-tolerance the north star allows for logits and 16-bit rows, 2 ulp of float32,
-is not used: the engine reproduces the reference's operation order.)
+scores, raw scores, final scores, row logsumexp and the NaN/+inf flags, from
+logits and 16-bit rows too (the engine reproduces the reference's operation
+order).
 """
 
 import os
@@ -85,9 +85,10 @@ def test_invalid_rows_flagged_only_when_read(hip, oracle):
     assert out["invalid"].tolist() == want["invalid"].tolist() == [0, 1, 1]
 
 
-# 16-bit rows have three row-pass kernels with identical results: the
-# pipelined one (the default; any V, rows at any 2-byte offset), the resident
-# one (V % 8 == 0) and the two-pass one. Each runs on the same inputs.
+# 16-bit rows have four row-pass kernels with identical results: the stream
+# one (7), the short-row one (8, up to 6144 entries), the two-pass one (0) and,
+# for bfloat16 logits with V % 8 == 0, the relay (5); a kernel that does not
+# apply falls back to the two-pass one. Each runs on the same inputs.
 _ROW_PASS_VOCABS = [8, 40, 255, 256, 257, 1000, 2047, 2048, 3000, 4104, 8200, 8201]
 
 
@@ -100,7 +101,7 @@ def row_pass(hip):
     hip.lib.dbs_hip_set_row_pass(-1)
 
 
-@pytest.mark.parametrize("kind", [2, 1, 0, 5])
+@pytest.mark.parametrize("kind", [7, 8, 0, 5])
 @pytest.mark.parametrize("seed", range(0, 30))
 def test_decode_16bit_row_passes(hip, oracle, row_pass, seed, kind):
     row_pass(kind)
@@ -108,11 +109,11 @@ def test_decode_16bit_row_passes(hip, oracle, row_pass, seed, kind):
     _check(hip, oracle, case)
 
 
-# Log-prob rows of every dtype take the one-read kernel where the row fits on
-# chip (the default) and the two-pass kernel otherwise; both run on the same
-# inputs, with the rows at every alignment (an element offset of 0-4 from the
-# allocation), vocabularies at the block and on-chip limits (fp32 rows up to
-# 40956 elements, 16-bit up to 81912), and one past them.
+# Log-prob rows of every dtype take the one-read kernel where a row fits its
+# registers; it and the two-pass kernel run on the same inputs, with the rows at
+# every alignment (an element offset of 0-4 from the allocation) and
+# vocabularies around its blocks (40 of 256 threads end at 40956 float32 and
+# 81912 16-bit entries; the longest rows it takes are in test_gpu_row_stream.py).
 _LOGPROB_VOCABS = [2, 7, 8, 255, 256, 257, 1000, 1021, 4097, 8192, 32000, 40956, 40957, 50257, 81912, 81913]
 
 
@@ -126,8 +127,8 @@ def test_decode_logprob_row_passes(hip, oracle, row_pass, seed, kind):
 
 @pytest.mark.parametrize("seed", range(0, 6))
 def test_decode_16bit_wide_beams(hip, oracle, seed):
-    """K > 64: no shortlist (every read row is rescanned); the row pass still
-    gives the logsumexp and the flags."""
+    """Some cases with K > 64, whose shortlists hold fewer entries than the
+    search keeps beams."""
     case = make_case(9500 + seed, big=True, dtypes=["bf16"], vocabs=[1000, 4104])
     _check(hip, oracle, case)
 
@@ -192,8 +193,8 @@ def test_logsumexp_table_edges(hip, oracle, row_pass, m, kind):
 @pytest.mark.parametrize("V,dtype", [(151936, "bf16"), (128256, "bf16"), (155648, "bf16"), (155656, "bf16"),
                                      (151936, "f16")])
 def test_decode_large_vocab_16bit(hip, oracle, V, dtype):
-    """Full-size vocabularies around the on-chip limit (155648 entries; one
-    more stripe falls back to the two-pass kernel)."""
+    """Full-size vocabularies around the relay kernel's limit (155648 entries;
+    one more stripe, and binary16, take the stream kernel)."""
     rng = np.random.default_rng(V % 1000 + 11)
     x = rng.normal(0.0, 3.0, size=(1, 3, 4, V)).astype(np.float32)
     x += (-1.1 * np.log(rng.permutation(V) + 1.0)).astype(np.float32)
@@ -211,7 +212,7 @@ def test_decode_large_vocab_16bit(hip, oracle, V, dtype):
 # stream that follows the row pass step by step; dbs_hip_set_decode_overlap:
 # 1 always, 0 never, -1 constrained decodes only). Every order gives the
 # oracle's bits, with every row-pass kernel, and no wait for a step gives up.
-@pytest.mark.parametrize("kind", [-1, 2, 0])
+@pytest.mark.parametrize("kind", [-1, 7, 0])
 @pytest.mark.parametrize("overlap", [1, 0, -1])
 @pytest.mark.parametrize("seed", range(0, 10))
 def test_decode_overlapped_select(hip, oracle, row_pass, seed, overlap, kind):
