@@ -334,9 +334,9 @@ size_t sync_bytes(int B, int T) {
 
 // The row pass, then the select pass. With several steps and at most half
 // the CUs taken by the select pass's workgroups (one per example), the select
-// pass can run alongside on a second stream, following the row pass step by
-// step: the row pass is queued first and never waits on the select pass, and
-// its rows are handed out by ticket, so it always progresses on the CUs left.
+// pass can run alongside, on two streams, following the row pass step by step:
+// the row pass never waits on the select pass, and its rows are handed out by
+// ticket, so it always progresses on the CUs left.
 // By default constrained decodes (n-gram blocking, repetition penalty) do (64 x
 // 128 x 5 x 50257 f16: 720 us of row pass and 433 of select pass take 837);
 // decodes whose row pass is the relay kernel (one workgroup per CU, the row on
@@ -344,11 +344,13 @@ size_t sync_bytes(int B, int T) {
 // 2.00 -> 1.89 ms, 16 x 128 x 8 x 128256 2.35 -> 1.75); and decodes with the
 // workgroup select pass when at most one example per 8 CUs lets the select
 // pass hold its CUs (16 x 64 x 64 x 32000 f32 2.73 -> 2.13 ms; shared CUs made
-// it 3.53 ms). The one-wavefront pass of an unconstrained decode ends sooner
-// after the stream and log-prob passes than beside them: 40 us of launches and
-// events, and rows that complete several per CU at a time, 100 us behind their
-// step (float32 and float16 logits; batches of 0.5 GB and more of bfloat16 or
-// log-probs would gain 5-15 %).
+// it 3.53 ms). The one-wavefront pass of an unconstrained decode runs after the
+// stream and log-prob passes: beside them it pays 40 us of launches and events,
+// and rows that complete several per CU at a time come 100 us behind their step,
+// so float32 and float16 logits and batches below 0.5 GB end sooner without.
+// (Larger batches of bfloat16 logits or log-probs measured 5-15 % faster beside
+// it, with dbs_hip_set_decode_overlap(1); the automatic choice has no rule for
+// them.)
 // *fault: the overlapped decode's fault word (non-zero once a select-pass
 // wait gave up), else null.
 hipError_t launch_decode(const DecodeParams& p0, const DecodeLayout& L, hipStream_t stream, char* ws,
